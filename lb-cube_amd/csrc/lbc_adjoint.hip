@@ -356,8 +356,7 @@ __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
     // XCD-aware block order as in the forward kernels (the reverse pulls share
     // block-edge lines the same way); each block keeps its own dJ/d omega_c
     // slot, indexed by the dispatch id, so a slot always sums the same cells
-    const uint32_t block = renumber_blocks<F::D, R>() ? xcd_block() : blockIdx.x;
-    const uint32_t cell = block * blockDim.x + threadIdx.x;
+    const uint32_t cell = ordered_block(c.order) * blockDim.x + threadIdx.x;
     double acc = 0.0;
     if (cell < c.count) {
         const CellCoord q = cell_coord(cell, c);
@@ -689,6 +688,8 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
                         int interval,
                         double omega_d, double omega_c_d, double k_d, double* J_out, R* gf, R* ga, R* gb,
                         double* djdwc_out, char* ws, hipStream_t st) {
+    LaunchShape sa = s;  // the adjoint's blocks
+    sa.cells.order = F::D == 2 && sizeof(RA) <= 4 ? kContiguousOrder : kDispatchOrder;
     using St = State<F, S, R>;
     using StA = State<F, S, RA>;
     const int storage = std::is_same<R, double>::value ? kF64 : kF32;
@@ -797,11 +798,11 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
             StA in(nu1, cells), out(nu0, cells);
             if (s.threads() <= 256)
                 hipLaunchKernelGGL((reactive_adjoint_kernel<F, S, R, RA, CT, 256>), s.grid, s.block, 0, st, fw.f,
-                                   fw.a, fw.b, in.f, in.a, in.b, out.f, out.a, out.b, s.cells, omega, wm, omega_c, k,
+                                   fw.a, fw.b, in.f, in.a, in.b, out.f, out.a, out.b, sa.cells, omega, wm, omega_c, k,
                                    part);
             else
                 hipLaunchKernelGGL((reactive_adjoint_kernel<F, S, R, RA, CT, 1024>), s.grid, s.block, 0, st, fw.f,
-                                   fw.a, fw.b, in.f, in.a, in.b, out.f, out.a, out.b, s.cells, omega, wm, omega_c, k,
+                                   fw.a, fw.b, in.f, in.a, in.b, out.f, out.a, out.b, sa.cells, omega, wm, omega_c, k,
                                    part);
             if ((e = hipGetLastError()) != hipSuccess) return e;
             std::swap(nu0, nu1);

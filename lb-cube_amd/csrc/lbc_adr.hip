@@ -27,8 +27,8 @@ namespace lbc {
 // TILED: the buffers stored in tiles (tile_layout), the fluid's spaced by
 // c.zgap and the species' by zgap_s, each `plane` cells per population and
 // tile; tiled grids keep the dispatch order of their blocks, as the fused
-// step's do.
-template <class F, class S, int ST, bool REACT, int MAXT, bool WIDE, bool TILED>
+// step's do.  NT: the store form.
+template <class F, class S, int ST, bool REACT, int MAXT, bool WIDE, bool TILED, bool NT>
 __global__ __launch_bounds__(MAXT) void scalar_step_kernel(
     const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
     const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b,
@@ -37,8 +37,7 @@ __global__ __launch_bounds__(MAXT) void scalar_step_kernel(
     typename Storage<ST>::R ref_b) {
     using St = Storage<ST>;
     using R = typename St::R;
-    const uint32_t block = (!TILED && renumber_blocks<S::D, typename Storage<ST>::S>()) ? xcd_block() : blockIdx.x;
-    const uint32_t cell = block * blockDim.x + threadIdx.x;
+    const uint32_t cell = (TILED ? blockIdx.x : ordered_block(c.order)) * blockDim.x + threadIdx.x;
     if (cell >= c.count) return;
     const CellCoord q = cell_coord(cell, c);
     const int x = q.x, y = q.y, z = q.z;
@@ -71,8 +70,9 @@ __global__ __launch_bounds__(MAXT) void scalar_step_kernel(
     const uint32_t scell = TILED ? pull.dst : cell;
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
-        St::store(at<WIDE>(plane_ptr(nxt_a, i, pl), scell), ga[i], R(S::w[i]) * ref_a);
-        if constexpr (REACT) St::store(at<WIDE>(plane_ptr(nxt_b, i, pl), scell), gb[i], R(S::w[i]) * ref_b);
+        St::template store<NT>(at<WIDE>(plane_ptr(nxt_a, i, pl), scell), ga[i], R(S::w[i]) * ref_a);
+        if constexpr (REACT)
+            St::template store<NT>(at<WIDE>(plane_ptr(nxt_b, i, pl), scell), gb[i], R(S::w[i]) * ref_b);
     }
 }
 
@@ -80,9 +80,9 @@ __global__ __launch_bounds__(MAXT) void scalar_step_kernel(
 // with the lattices' Q, so the fluid and the species take pulls of their own;
 // otherwise one pull serves all three.  Tiled 2D grids keep the dispatch
 // order of their blocks (measured at 2048^2, tiles of 4 rows: FP32 39.0k
-// MLUPS against 37.2k with the XCD renumbering, FP16 deviation form 76.0k
-// against 69.5k), while the reference's planes gain from the renumbering.
-template <class F, int CT, class S, int ST, bool FAST, int MAXT, bool WIDE, bool TILED>
+// MLUPS against 37.2k with one contiguous run per XCD, FP16 deviation form
+// 76.0k against 69.5k), while the reference's planes gain from runs.
+template <class F, int CT, class S, int ST, bool FAST, int MAXT, bool WIDE, bool TILED, bool NT>
 __global__ __launch_bounds__(MAXT) void reactive_fused_kernel(
     const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
     const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
@@ -90,9 +90,7 @@ __global__ __launch_bounds__(MAXT) void reactive_fused_kernel(
     uint32_t plane, uint32_t zgap_s, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
     typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react, typename Storage<ST>::R ref_a,
     typename Storage<ST>::R ref_b) {
-    const uint32_t block =
-        (!TILED && renumber_blocks<F::D, typename Storage<ST>::S>()) ? xcd_block() : blockIdx.x;
-    const uint32_t p = block * blockDim.x + threadIdx.x;
+    const uint32_t p = (TILED ? blockIdx.x : ordered_block(c.order)) * blockDim.x + threadIdx.x;
     if (p >= c.count) return;
     const CellCoord q = cell_coord(p, c);
     Pull pf(p, q.x, q.y, q.z, static_cast<int>(c.nx), static_cast<int>(c.ny), static_cast<int>(c.nz));
@@ -105,11 +103,11 @@ __global__ __launch_bounds__(MAXT) void reactive_fused_kernel(
     // arithmetic of the untiled kernels has always seen it)
     const size_t pl = TILED ? plane : c.count;
     if constexpr (FAST)
-        reactive_cell_fast<F, CT, S, ST, WIDE>(cur_f, nxt_f, cur_a, nxt_a, cur_b, nxt_b, pf, ps, pl, omega,
-                                               omega_minus, omega_c, k_react, ref_a, ref_b);
+        reactive_cell_fast<F, CT, S, ST, WIDE, NT>(cur_f, nxt_f, cur_a, nxt_a, cur_b, nxt_b, pf, ps, pl, omega,
+                                                   omega_minus, omega_c, k_react, ref_a, ref_b);
     else
-        reactive_cell<F, CT, S, ST, WIDE>(cur_f, nxt_f, cur_a, nxt_a, cur_b, nxt_b, pf, ps, pl, omega, omega_minus,
-                                          omega_c, k_react, ref_a, ref_b);
+        reactive_cell<F, CT, S, ST, WIDE, NT>(cur_f, nxt_f, cur_a, nxt_a, cur_b, nxt_b, pf, ps, pl, omega,
+                                              omega_minus, omega_c, k_react, ref_a, ref_b);
 }
 
 // The fused step's access pattern alone: every fluid and species population
@@ -117,15 +115,14 @@ __global__ __launch_bounds__(MAXT) void reactive_fused_kernel(
 // kernel's addressing, block order, launch shape and residency and no
 // arithmetic.  Its rate is the ceiling of the fused step's memory pattern on
 // the same buffers (the reference's planes or tiles).
-template <class F, class S, int ST, int MAXT, bool WIDE, bool TILED, bool SHIFT>
+template <class F, class S, int ST, int MAXT, bool WIDE, bool TILED, bool SHIFT, bool NT>
 __global__ __launch_bounds__(MAXT) void reactive_pull_kernel(
     const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
     const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
     const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b, Cells c,
     uint32_t plane, uint32_t zgap_s) {
     using T = typename Storage<ST>::S;
-    const uint32_t block = (!TILED && renumber_blocks<F::D, T>()) ? xcd_block() : blockIdx.x;
-    const uint32_t p = block * blockDim.x + threadIdx.x;
+    const uint32_t p = (TILED ? blockIdx.x : ordered_block(c.order)) * blockDim.x + threadIdx.x;
     if (p >= c.count) return;
     const CellCoord q = cell_coord(p, c);
     Pull pf(p, q.x, q.y, q.z, static_cast<int>(c.nx), static_cast<int>(c.ny), static_cast<int>(c.nz));
@@ -140,7 +137,7 @@ __global__ __launch_bounds__(MAXT) void reactive_pull_kernel(
     for (int i = 0; i < F::Q; ++i)
         v[i] = get(at<WIDE>(plane_ptr(cur_f, i, pl), SHIFT ? pf.src(F::cx[i], F::cy[i], F::cz[i]) : pf.dst));
 #pragma unroll
-    for (int i = 0; i < F::Q; ++i) put(at<WIDE>(plane_ptr(nxt_f, i, pl), pf.dst), v[i]);
+    for (int i = 0; i < F::Q; ++i) put<NT>(at<WIDE>(plane_ptr(nxt_f, i, pl), pf.dst), v[i]);
     T va[S::Q], vb[S::Q];
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
@@ -150,8 +147,8 @@ __global__ __launch_bounds__(MAXT) void reactive_pull_kernel(
     }
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
-        put(at<WIDE>(plane_ptr(nxt_a, i, pl), ps.dst), va[i]);
-        put(at<WIDE>(plane_ptr(nxt_b, i, pl), ps.dst), vb[i]);
+        put<NT>(at<WIDE>(plane_ptr(nxt_a, i, pl), ps.dst), va[i]);
+        put<NT>(at<WIDE>(plane_ptr(nxt_b, i, pl), ps.dst), vb[i]);
     }
 }
 
@@ -166,8 +163,38 @@ template <int D, int ST, bool FUSED> constexpr bool capped_residency_adr() {
     return D == 3 && (ST == kF32 || (FUSED && ST == kF16));
 }
 
+// The store form and the block order (plan_traffic) of a step whose time loop
+// holds `planes` population planes and that writes at `bases`.  Streaming
+// grids whose loop takes up to kWindowBytes run contiguously (fused step:
+// D2Q9 MRT FP32 at 2048^2, 637 MB, 112 us against 120 in dispatch order and
+// 118 in runs of 8; D3Q19 FP32 at 128^3, 554 MB, 103 against 110 us; fluid and
+// reaction step at 1448^2 FP64 139 against 144 us); above it contiguous runs
+// lose (2048 x 4096 FP32, 1.3 GB, 240 against 232 us; 192^3 FP32 363 against
+// 344 us).  Tiled buffers and planes of more than 4 GiB stream, in dispatch
+// order.
+constexpr uint64_t kWindowBytes = 730ull << 20;
+
+template <int D, class T>
+Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t planes) {
+    const uint64_t footprint = planes * s.cells.count * sizeof(T);
+    Traffic t = plan_traffic<D, T>(s, bases, s.cells.count, footprint);
+    if (t.streaming && footprint <= kWindowBytes) t.order = kContiguousOrder;
+    if (tiled || wide_planes<T>(s)) t = Traffic{true, kDispatchOrder};
+    s.cells.order = t.order;
+    return t;
+}
+
+// Calls go<WIDE, TILED, NT> of the instantiations a launch may take.
+template <class Go> void pick_form(bool wide, bool tiled, bool streaming, Go go) {
+    using Y = std::true_type;
+    using N = std::false_type;
+    if (tiled) wide ? go(Y{}, Y{}, Y{}) : go(N{}, Y{}, Y{});
+    else if (wide) go(Y{}, N{}, Y{});
+    else streaming ? go(N{}, N{}, Y{}) : go(N{}, N{}, N{});
+}
+
 template <class F, class S, int ST, bool REACT>
-hipError_t launch_scalar(const void* ca, void* na, const void* cb, void* nb, const void* cf, const LaunchShape& s,
+hipError_t launch_scalar(const void* ca, void* na, const void* cb, void* nb, const void* cf, LaunchShape s,
                          double omega_c, double param, double ref_a, double ref_b, hipStream_t stream) {
     using St = Storage<ST>;
     using T = typename St::S;
@@ -177,6 +204,8 @@ hipError_t launch_scalar(const void* ca, void* na, const void* cb, void* nb, con
     const bool tiled = s.cells.zgap != 0 && (S::D == 3 || s.cells.tiles > 1);
     const uint32_t plane = tiled ? s.cells.zgap / (F::Q - 1) : s.cells.count;
     const uint32_t zgap_s = tiled ? (S::Q - 1) * plane : 0u;
+    const Traffic t = adr_traffic<S::D, T>(s, tiled, address(na) | (REACT ? address(nb) : 0),
+                                           2 * F::Q + (REACT ? 4 : 2) * S::Q);
     const uint32_t lds = capped_residency_adr<S::D, ST, false>() ? capped_lds(s.threads()) : 0;
     auto args = [&](auto kern) {
         hipLaunchKernelGGL(kern, s.grid, s.block, lds, stream, static_cast<const T*>(ca), static_cast<T*>(na),
@@ -184,17 +213,11 @@ hipError_t launch_scalar(const void* ca, void* na, const void* cb, void* nb, con
                            zgap_s, static_cast<R>(omega_c), static_cast<R>(param), static_cast<R>(ref_a),
                            static_cast<R>(ref_b));
     };
-    const bool wide = wide_planes<T>(s);
-    auto pick = [&](auto tl) {
-        constexpr bool TL = decltype(tl)::value;
-        if (s.threads() <= 256)
-            wide ? args(scalar_step_kernel<F, S, ST, REACT, 256, true, TL>)
-                 : args(scalar_step_kernel<F, S, ST, REACT, 256, false, TL>);
-        else
-            wide ? args(scalar_step_kernel<F, S, ST, REACT, 1024, true, TL>)
-                 : args(scalar_step_kernel<F, S, ST, REACT, 1024, false, TL>);
-    };
-    tiled ? pick(std::true_type{}) : pick(std::false_type{});
+    pick_form(wide_planes<T>(s), tiled, t.streaming, [&](auto w, auto tl, auto nt) {
+        constexpr bool W = decltype(w)::value, TL = decltype(tl)::value, NT = decltype(nt)::value;
+        s.threads() <= 256 ? args(scalar_step_kernel<F, S, ST, REACT, 256, W, TL, NT>)
+                           : args(scalar_step_kernel<F, S, ST, REACT, 1024, W, TL, NT>);
+    });
     return hipGetLastError();
 }
 
@@ -228,7 +251,7 @@ hipError_t scalar_dispatch(int fl, int sl, int storage, const void* ca, void* na
 // species' gap follows from their Q.
 template <class F, int CT, class S, int ST, bool FAST>
 hipError_t launch_fused(const void* cf, void* nf, const void* ca, void* na, const void* cb, void* nb,
-                        const LaunchShape& s, double omega, double omega_c, double k, double ra, double rb,
+                        LaunchShape s, double omega, double omega_c, double k, double ra, double rb,
                         hipStream_t stream) {
     // one 2D tile holding every row is the reference's planes
     const bool tiled = s.cells.zgap != 0 && (F::D == 3 || s.cells.tiles > 1);
@@ -239,6 +262,7 @@ hipError_t launch_fused(const void* cf, void* nf, const void* ca, void* na, cons
     using R = typename St::R;
     const R w = static_cast<R>(omega);
     const R wm = CT == kTRT ? trt_omega_minus<R>(w) : R(0);
+    const Traffic t = adr_traffic<F::D, T>(s, tiled, address(nf) | address(na) | address(nb), 2 * F::Q + 4 * S::Q);
     const uint32_t lds = capped_residency_adr<F::D, ST, true>() ? capped_lds(s.threads()) : 0;
     auto args = [&](auto kern) {
         hipLaunchKernelGGL(kern, s.grid, s.block, lds, stream, static_cast<const T*>(cf), static_cast<T*>(nf),
@@ -246,17 +270,11 @@ hipError_t launch_fused(const void* cf, void* nf, const void* ca, void* na, cons
                            static_cast<T*>(nb), s.cells, plane, zgap_s, w, wm, static_cast<R>(omega_c),
                            static_cast<R>(k), static_cast<R>(ra), static_cast<R>(rb));
     };
-    const bool wide = wide_planes<T>(s);
-    auto pick = [&](auto tiled) {
-        constexpr bool TL = decltype(tiled)::value;
-        if (s.threads() <= 256)
-            wide ? args(reactive_fused_kernel<F, CT, S, ST, FAST, 256, true, TL>)
-                 : args(reactive_fused_kernel<F, CT, S, ST, FAST, 256, false, TL>);
-        else
-            wide ? args(reactive_fused_kernel<F, CT, S, ST, FAST, 1024, true, TL>)
-                 : args(reactive_fused_kernel<F, CT, S, ST, FAST, 1024, false, TL>);
-    };
-    tiled ? pick(std::true_type{}) : pick(std::false_type{});
+    pick_form(wide_planes<T>(s), tiled, t.streaming, [&](auto wd, auto tl, auto nt) {
+        constexpr bool W = decltype(wd)::value, TL = decltype(tl)::value, NT = decltype(nt)::value;
+        s.threads() <= 256 ? args(reactive_fused_kernel<F, CT, S, ST, FAST, 256, W, TL, NT>)
+                           : args(reactive_fused_kernel<F, CT, S, ST, FAST, 1024, W, TL, NT>);
+    });
     return hipGetLastError();
 }
 
@@ -291,28 +309,23 @@ hipError_t fused_by_collision(int collision, int storage, bool fast, const void*
 
 template <class F, class S, int ST, bool SHIFT>
 hipError_t launch_reactive_pull(const void* cf, void* nf, const void* ca, void* na, const void* cb, void* nb,
-                                const LaunchShape& s, hipStream_t stream) {
+                                LaunchShape s, hipStream_t stream) {
     using T = typename Storage<ST>::S;
     const bool tiled = s.cells.zgap != 0 && (F::D == 3 || s.cells.tiles > 1);
     const uint32_t plane = tiled ? s.cells.zgap / (F::Q - 1) : s.cells.count;
     const uint32_t zgap_s = tiled ? (S::Q - 1) * plane : 0u;
+    const Traffic t = adr_traffic<F::D, T>(s, tiled, address(nf) | address(na) | address(nb), 2 * F::Q + 4 * S::Q);
     const uint32_t lds = capped_residency_adr<F::D, ST, true>() ? capped_lds(s.threads()) : 0;
     auto args = [&](auto kern) {
         hipLaunchKernelGGL(kern, s.grid, s.block, lds, stream, static_cast<const T*>(cf), static_cast<T*>(nf),
                            static_cast<const T*>(ca), static_cast<T*>(na), static_cast<const T*>(cb),
                            static_cast<T*>(nb), s.cells, plane, zgap_s);
     };
-    const bool wide = wide_planes<T>(s);
-    auto pick = [&](auto tl) {
-        constexpr bool TL = decltype(tl)::value;
-        if (s.threads() <= 256)
-            wide ? args(reactive_pull_kernel<F, S, ST, 256, true, TL, SHIFT>)
-                 : args(reactive_pull_kernel<F, S, ST, 256, false, TL, SHIFT>);
-        else
-            wide ? args(reactive_pull_kernel<F, S, ST, 1024, true, TL, SHIFT>)
-                 : args(reactive_pull_kernel<F, S, ST, 1024, false, TL, SHIFT>);
-    };
-    tiled ? pick(std::true_type{}) : pick(std::false_type{});
+    pick_form(wide_planes<T>(s), tiled, t.streaming, [&](auto wd, auto tl, auto nt) {
+        constexpr bool W = decltype(wd)::value, TL = decltype(tl)::value, NT = decltype(nt)::value;
+        s.threads() <= 256 ? args(reactive_pull_kernel<F, S, ST, 256, W, TL, SHIFT, NT>)
+                           : args(reactive_pull_kernel<F, S, ST, 1024, W, TL, SHIFT, NT>);
+    });
     return hipGetLastError();
 }
 

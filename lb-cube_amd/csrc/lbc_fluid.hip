@@ -11,6 +11,8 @@
 // (per-lane offsets 32-bit, or 64-bit for planes of more than 4 GiB).
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "../../include/lbcube.h"
 #include "lbc_fast.hpp"
 #include "lbc_launch.hpp"
@@ -23,20 +25,17 @@ namespace lbc {
 // FAST selects the deviation-form arithmetic (lbc_fast.hpp) behind
 // LBC_FLAG_FAST: BGK, TRT and MRT on every lattice; RLBM always evaluates the
 // reference's order.  WIDE: 64-bit per-lane addresses, for planes of more than
-// 4 GiB.
+// 4 GiB.  NT: the store form.
 // `plane`: elements from one population plane to the next (the cell count for
 // the reference's contiguous [Q][Z][Y][X] buffers; larger for pitched ones).
-template <class L, int CT, int ST, bool FAST, int MAXT, bool WIDE>
+template <class L, int CT, int ST, bool FAST, int MAXT, bool WIDE, bool NT>
 __global__ __launch_bounds__(MAXT) void fluid_step_kernel(const typename Storage<ST>::S* __restrict__ cur,
                                                           typename Storage<ST>::S* __restrict__ nxt, Cells c,
                                                           size_t plane, typename Storage<ST>::R omega,
                                                           typename Storage<ST>::R omega_minus) {
     using St = Storage<ST>;
     using R = typename St::R;
-    // tiled 2D grids keep the dispatch order (as the fused reactive kernel)
-    const uint32_t block =
-        (renumber_blocks<L::D, typename Storage<ST>::S>() && c.tiles == 1) ? xcd_block() : blockIdx.x;
-    const uint32_t dst = block * blockDim.x + threadIdx.x;
+    const uint32_t dst = ordered_block(c.order) * blockDim.x + threadIdx.x;
     if (dst >= c.count) return;
     const CellCoord q = cell_coord(dst, c);
     const Pull pull = locate<L::D>(dst, q, c, c.zgap);
@@ -49,7 +48,7 @@ __global__ __launch_bounds__(MAXT) void fluid_step_kernel(const typename Storage
             f[i] = St::load_dev(at<WIDE>(plane_ptr(cur, i, plane), src), R(L::w[i]));
         }
         collide_dev<L, CT, R>(f, omega, omega_minus, [&](int i, R v) {
-            St::store_dev(at<WIDE>(plane_ptr_opaque(nxt, i, plane), cell), v, R(L::w[i]));
+            St::template store_dev<NT>(at<WIDE>(plane_ptr_opaque(nxt, i, plane), cell), v, R(L::w[i]));
         });
     } else {
 #pragma unroll
@@ -59,7 +58,8 @@ __global__ __launch_bounds__(MAXT) void fluid_step_kernel(const typename Storage
             f[i] = St::load(at<WIDE>(plane_ptr(cur, i, plane), src), off);
         }
         collide_cell<L, CT, R>(f, omega, omega_minus, [&](int i, R v) {
-            St::store(at<WIDE>(plane_ptr_opaque(nxt, i, plane), cell), v, kOffsetStorage<ST> ? R(L::w[i]) : R(0));
+            St::template store<NT>(at<WIDE>(plane_ptr_opaque(nxt, i, plane), cell), v,
+                                   kOffsetStorage<ST> ? R(L::w[i]) : R(0));
         });
     }
 }
@@ -130,13 +130,11 @@ __global__ __launch_bounds__(MAXT) void fluid_step_mfma_kernel(const uint16_t* _
 // pattern: the same 2 Q streams with the x-shifted pulls, without arithmetic.
 // SHIFT = false: the same 2 Q plane streams read without the shifts
 // (next[i][x] = cur[i][x]), the ceiling of the plane streams themselves.
-template <class L, int ST, int MAXT, bool WIDE, bool SHIFT = true>
+template <class L, int ST, int MAXT, bool WIDE, bool SHIFT, bool NT>
 __global__ __launch_bounds__(MAXT) void pull_stream_kernel(const typename Storage<ST>::S* __restrict__ cur,
                                                            typename Storage<ST>::S* __restrict__ nxt, Cells c,
                                                            size_t plane) {
-    const uint32_t block =
-        (renumber_blocks<L::D, typename Storage<ST>::S>() && c.tiles == 1) ? xcd_block() : blockIdx.x;
-    const uint32_t dst = block * blockDim.x + threadIdx.x;
+    const uint32_t dst = ordered_block(c.order) * blockDim.x + threadIdx.x;
     if (dst >= c.count) return;
     const CellCoord q = cell_coord(dst, c);
     const Pull pull = locate<L::D>(dst, q, c, c.zgap);
@@ -146,7 +144,7 @@ __global__ __launch_bounds__(MAXT) void pull_stream_kernel(const typename Storag
     for (int i = 0; i < L::Q; ++i)
         v[i] = get(at<WIDE>(plane_ptr(cur, i, plane), SHIFT ? pull.src(L::cx[i], L::cy[i], L::cz[i]) : cell));
 #pragma unroll
-    for (int i = 0; i < L::Q; ++i) put(at<WIDE>(plane_ptr_opaque(nxt, i, plane), cell), v[i]);
+    for (int i = 0; i < L::Q; ++i) put<NT>(at<WIDE>(plane_ptr_opaque(nxt, i, plane), cell), v[i]);
 }
 
 // Kernels that run faster with residency capped at kCappedWavesPerCu (measured
@@ -176,24 +174,37 @@ template <class L, int CT, int ST, bool FAST> constexpr uint32_t capped_waves() 
     return (L::Q == 19 && ST == kF16 && FAST) ? 24u : kCappedWavesPerCu;
 }
 
+// The store form and the block order of a fluid step.  Tiles of fewer rows
+// than a slab and planes of more than 4 GiB stream, in dispatch order.
+template <class L, class S> Traffic fluid_traffic(LaunchShape& s, const void* nxt, uint64_t plane) {
+    Traffic t = plan_traffic<L::D, S>(s, address(nxt), plane, 2ull * L::Q * s.cells.count * sizeof(S));
+    if (s.cells.tiles > 1 || wide_planes<S>(s)) t = Traffic{true, kDispatchOrder};
+    s.cells.order = t.order;
+    return t;
+}
+
 template <class L, int CT, int ST, bool FAST>
-hipError_t launch_fluid(const void* cur, void* nxt, const LaunchShape& s, uint64_t plane, double omega,
+hipError_t launch_fluid(const void* cur, void* nxt, LaunchShape s, uint64_t plane, double omega,
                         hipStream_t stream) {
     using St = Storage<ST>;
     using R = typename St::R;
     const R w = static_cast<R>(omega);
     const R wm = CT == kTRT ? trt_omega_minus<R>(w) : R(0);
+    const Traffic t = fluid_traffic<L, typename St::S>(s, nxt, plane);
     const uint32_t lds =
         capped_residency<L, CT, ST, FAST>() ? capped_lds(s.threads(), capped_waves<L, CT, ST, FAST>()) : 0;
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, s.grid, s.block, lds, stream, static_cast<const typename St::S*>(cur),
                            static_cast<typename St::S*>(nxt), s.cells, static_cast<size_t>(plane), w, wm);
     };
-    const bool wide = wide_planes<typename St::S>(s);
-    if (s.threads() <= 256)
-        wide ? go(fluid_step_kernel<L, CT, ST, FAST, 256, true>) : go(fluid_step_kernel<L, CT, ST, FAST, 256, false>);
-    else
-        wide ? go(fluid_step_kernel<L, CT, ST, FAST, 1024, true>) : go(fluid_step_kernel<L, CT, ST, FAST, 1024, false>);
+    auto pick = [&](auto maxt) {
+        constexpr int M = decltype(maxt)::value;
+        if (wide_planes<typename St::S>(s)) go(fluid_step_kernel<L, CT, ST, FAST, M, true, true>);
+        else if (t.streaming) go(fluid_step_kernel<L, CT, ST, FAST, M, false, true>);
+        else go(fluid_step_kernel<L, CT, ST, FAST, M, false, false>);
+    };
+    if (s.threads() <= 256) pick(std::integral_constant<int, 256>{});
+    else pick(std::integral_constant<int, 1024>{});
     return hipGetLastError();
 }
 
@@ -259,22 +270,27 @@ hipError_t dispatch_mfma(int lattice, int collision, int storage, uint32_t flags
                            : launch_fluid_mfma<D3Q27, kBF16>(cur, nxt, s, plane, omega, st);
 }
 
-// The pull-streaming step shares the residency of the TRT step it bounds.
+// The pull-streaming step shares the residency and the traffic plan of the TRT
+// step it bounds.
 template <class L, int ST, bool SHIFT>
-hipError_t launch_stream(const void* cur, void* nxt, const LaunchShape& s, uint64_t plane, hipStream_t stream) {
+hipError_t launch_stream(const void* cur, void* nxt, LaunchShape s, uint64_t plane, hipStream_t stream) {
     using S = typename Storage<ST>::S;
     constexpr bool kFast = kOffsetStorage<ST>;
+    const Traffic t = fluid_traffic<L, S>(s, nxt, plane);
     const uint32_t lds =
         capped_residency<L, kTRT, ST, kFast>() ? capped_lds(s.threads(), capped_waves<L, kTRT, ST, kFast>()) : 0;
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, s.grid, s.block, lds, stream, static_cast<const S*>(cur), static_cast<S*>(nxt),
                            s.cells, static_cast<size_t>(plane));
     };
-    const bool wide = wide_planes<S>(s);
-    if (s.threads() <= 256)
-        wide ? go(pull_stream_kernel<L, ST, 256, true, SHIFT>) : go(pull_stream_kernel<L, ST, 256, false, SHIFT>);
-    else
-        wide ? go(pull_stream_kernel<L, ST, 1024, true, SHIFT>) : go(pull_stream_kernel<L, ST, 1024, false, SHIFT>);
+    auto pick = [&](auto maxt) {
+        constexpr int M = decltype(maxt)::value;
+        if (wide_planes<S>(s)) go(pull_stream_kernel<L, ST, M, true, SHIFT, true>);
+        else if (t.streaming) go(pull_stream_kernel<L, ST, M, false, SHIFT, true>);
+        else go(pull_stream_kernel<L, ST, M, false, SHIFT, false>);
+    };
+    if (s.threads() <= 256) pick(std::integral_constant<int, 256>{});
+    else pick(std::integral_constant<int, 1024>{});
     return hipGetLastError();
 }
 

@@ -67,11 +67,16 @@ struct Cells {
     uint32_t zgap;
     uint32_t rows, tiles;
     FastDiv by_rows;
+    uint32_t order;  // of the blocks: ordered_block
 };
 
 struct CellCoord {
     int x, y, z;
 };
+
+// Block orders (ordered_block, below).
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kDispatchOrder = 0, kContiguousOrder = 31;
 
 __device__ __forceinline__ CellCoord cell_coord(uint32_t p, const Cells& c) {
     const uint32_t row = fast_div(p, c.by_nx);
@@ -164,7 +169,7 @@ inline hipError_t make_shape(bool two_d, uint64_t nx, uint64_t ny, uint64_t nz, 
     s.cells = Cells{static_cast<uint32_t>(nx), static_cast<uint32_t>(ny), static_cast<uint32_t>(nz),
                     static_cast<uint32_t>(count), make_fastdiv(static_cast<uint32_t>(nx)),
                     make_fastdiv(static_cast<uint32_t>(ny)), 0u, static_cast<uint32_t>(ny), 1u,
-                    make_fastdiv(static_cast<uint32_t>(ny))};
+                    make_fastdiv(static_cast<uint32_t>(ny)), kDispatchOrder};
     return hipSuccess;
 }
 
@@ -191,6 +196,8 @@ inline hipError_t tile_layout(bool two_d, uint64_t rows, int q_max, LaunchShape&
     c.zgap = static_cast<uint32_t>((q_max - 1) * plane);
     return hipSuccess;
 }
+
+inline uint64_t address(const void* p) { return reinterpret_cast<uint64_t>(p); }
 
 inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
@@ -239,31 +246,86 @@ inline uint32_t capped_lds(uint32_t threads, uint32_t waves = kCappedWavesPerCu)
 
 // The dispatcher hands workgroup b to XCD b % 8 (8 XCDs, each with its own
 // L2).  Blocks numbered linearly over the cells share the cache lines at their
-// x edges with their neighbours, so with that dispatch every edge line is
-// fetched into two L2s: +6.6% of the reads of a 2D FP32 reactive step, +13% in
-// FP16 (rocprofv3 FETCH_SIZE).  This renumbering gives each XCD one contiguous
-// run of blocks instead (a bijection for any grid size: XCDs x < nb % 8 take
-// one block more).  3D grids at 256^3 and above have whole rows per block and
-// no such lines, so only the 2D single-domain kernels use it (measured on the
-// 2048^2 reactive step: FETCH_SIZE back to the algorithmic bytes, +3.5% FP32,
-// +4% FP16).  The ensemble kernel keeps the dispatch order (renumbered, its
-// 512 instances ran 12% slower), and so do 3D grids whose rows split blocks
-// (renumbered, D3Q19 and D3Q27 at 384^3 ran 7-8% slower: each XCD's separate
-// window of the 38 streams costs more than the edge lines it saves).
-constexpr uint32_t kXcds = 8;
+// x edges with their neighbours, so in that dispatch order every edge line is
+// fetched into two L2s (+6.6% of the reads of a 2D FP32 reactive step at
+// 2048^2, +13% in FP16: rocprofv3 FETCH_SIZE), and an edge line that two
+// blocks write leaves two L2s in parts.  Renumbering the blocks gives each XCD
+// runs of consecutive ones.  kContiguousOrder: one run per XCD (a bijection
+// for any grid size: XCDs x < nb % 8 take one block more).  1 <= order < 31:
+// runs of 2^order blocks, eight runs (one per XCD) after another; the blocks
+// past the last whole group of eight runs keep the dispatch order.
+// The block that the dispatcher's block b of nb works on.
+__host__ __device__ __forceinline__ uint32_t block_at(uint32_t b, uint32_t nb, uint32_t order) {
+    if (order == kDispatchOrder) return b;
+    if (order == kContiguousOrder) {
+        const uint32_t q = nb / kXcds, r = nb % kXcds;
+        const uint32_t x = b % kXcds, slot = b / kXcds;
+        return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + slot;
+    }
+    const uint32_t group = kXcds << order;
+    const uint32_t first = b & ~(group - 1u);
+    if (nb - first < group) return b;
+    const uint32_t r = b - first;
+    return first + ((r % kXcds) << order) + r / kXcds;
+}
 
-// Where the renumbering pays (measured, 2048^2 reactive step): 2D grids with
-// elements of at most 4 bytes, whose 256-cell blocks span 8 lines per plane
-// (FP32) or 4 (FP16), so an edge line is 1/8 or 1/4 of a block's reads.  With
-// FP64 (16 lines per block) the saving is half as large and the renumbered
-// FP64 step ran 5% slower.
-template <int D, class S> __host__ __device__ constexpr bool renumber_blocks() { return D == 2 && sizeof(S) <= 4; }
+__device__ __forceinline__ uint32_t ordered_block(uint32_t order) { return block_at(blockIdx.x, gridDim.x, order); }
 
-__device__ __forceinline__ uint32_t xcd_block() {
-    const uint32_t nb = gridDim.x, b = blockIdx.x;
-    const uint32_t q = nb / kXcds, r = nb % kXcds;
-    const uint32_t x = b % kXcds, slot = b / kXcds;
-    return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + slot;
+// How a launch moves its populations: streaming or ordinary stores, and the
+// order of its blocks.
+struct Traffic {
+    bool streaming;
+    uint32_t order;
+};
+
+// Two levels of populations up to the size of the memory-side cache (256 MiB)
+// stay there from one step of a time loop to the next, so ordinary stores win.
+// D3Q19 TRT, streaming -> ordinary: 64^3 FP64 (80 MB) 16.1 -> 13.1 us, 112^3
+// FP32 (213 MB) 46.1 -> 33.9 us; 2D FP32 512^2 5.8 -> 3.9 us, 1448^2 (151 MB)
+// 28.2 -> 22.8 us.  Above it they gain little or lose: 128^3 FP32 (319 MB) 62.5
+// -> 58.3 us, 112^3 FP64 (427 MB) 79.8 -> 82.1 us, 160^3 FP32 (623 MB) 116 ->
+// 120 us, 256^3 FP32 425 -> 450 us, and a step whose output is not read next
+// pays for what they displace (128^3 FP32 47 -> 61 us).
+constexpr uint64_t kCachedBytes = 256ull << 20;
+
+// Streaming stores need every wave to write whole 64-byte sectors: the planes
+// `plane` elements apart and the base both on multiples of 64 bytes.  Where
+// they are not, each wave writes parts of two lines per plane, and a streaming
+// store sends them on before the neighbouring wave's part arrives: D3Q27 TRT
+// FP32 at 253 x 191 x 167 ran 427 us against 385 us with ordinary stores, and
+// 346 us with the blocks also in runs of 32 (the parts at the blocks' edges
+// then meet in one L2); D3Q19 TRT FP16 at 301 x 217 x 185 271, 230 and 194 us.
+//
+// The order, by what was measured (256-work-item blocks):
+//  - ordinary stores, 3D: runs of 32 (runs of 8 to 64 are within 2%).
+//  - ordinary stores, 2D, cache-resident: contiguous (D2Q9 FP64 at 512^2 9.2
+//    us in dispatch order, 7.1 us; FP32 at 1001 x 701 10.3 -> 9.0 us); larger
+//    2D grids runs of 32 (FP32 at 4095 x 2047 120 -> 109 us, contiguous 120).
+//  - streaming stores, 2D: contiguous up to kContiguousBytes (FP32 at 2048^2,
+//    302 MB, 62.6 us in dispatch order, 61.0 in runs of 8, 55.0 contiguous; FP64
+//    at 1448^2 58.4 -> 54.0 us), above it runs of 8 up to 4 bytes per element
+//    (FP32 at 4096 x 2048 107 us in dispatch order, 111 contiguous, 102 in
+//    runs) and FP64 in dispatch order (206 us, 210 in runs).
+//  - streaming stores, 3D: FP32 in dispatch order (256^3 425 us, in runs of 8
+//    446 us: each XCD's separate window of the 38 streams costs more than the
+//    edge lines save), the other formats in runs of 8 (D3Q19 FP16 at 256^3 223
+//    -> 212 us, BF16 at 256 x 256 x 200 193 -> 185 us, FP64 at 128^3 127 -> 118
+//    us, at 192^3 level).
+//
+// bases: the addresses of the buffers written, ORed; footprint: the bytes of
+// the buffers the step reads and writes.
+constexpr uint64_t kContiguousBytes = 350ull << 20;
+
+template <int D, class S>
+Traffic plan_traffic(const LaunchShape& s, uint64_t bases, uint64_t plane, uint64_t footprint) {
+    const uint64_t misaligned = (bases | plane * sizeof(S) | static_cast<uint64_t>(s.cells.zgap) * sizeof(S)) % 64;
+    const bool cached = footprint <= kCachedBytes;
+    if (!cached && misaligned == 0) {
+        if (D == 2 && footprint <= kContiguousBytes) return Traffic{true, kContiguousOrder};
+        if (D == 2) return Traffic{true, sizeof(S) <= 4 ? 3u : kDispatchOrder};
+        return Traffic{true, sizeof(S) == 4 ? kDispatchOrder : 3u};
+    }
+    return Traffic{false, D == 2 && footprint <= kContiguousBytes ? kContiguousOrder : 5u};
 }
 
 }  // namespace lbc

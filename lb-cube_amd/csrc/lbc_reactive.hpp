@@ -12,14 +12,15 @@ namespace lbc {
 // periodic sources in the fluid planes and `ps` in the species planes (the
 // same pull unless the buffers are stored in tiles, whose gaps differ with the
 // lattices' Q), `plane` is the element stride between population planes;
-// WIDE selects 64-bit per-lane addresses (planes of more than 4 GiB).
+// WIDE selects 64-bit per-lane addresses (planes of more than 4 GiB), NT the
+// store form.
 // The reaction step of the reference reads the fluid populations that the
 // fluid step has just written
 // at the same cell (src/simulate_reaction.cpp:527-541); here they are still in
 // registers.  With reduced-precision storage they are passed through the
 // storage rounding first, so the velocity is the one the unfused pair sees.
 // Shared by the single-domain kernel below and the ensemble kernel.
-template <class F, int CT, class S, int ST, bool WIDE = false>
+template <class F, int CT, class S, int ST, bool WIDE = false, bool NT = true>
 __device__ __forceinline__ void reactive_cell(const typename Storage<ST>::S* __restrict__ cur_f,
                                               typename Storage<ST>::S* __restrict__ nxt_f,
                                               const typename Storage<ST>::S* __restrict__ cur_a,
@@ -40,7 +41,7 @@ __device__ __forceinline__ void reactive_cell(const typename Storage<ST>::S* __r
         f[i] = St::load(at<WIDE>(plane_ptr(cur_f, i, plane), src), kOffsetStorage<ST> ? R(F::w[i]) : R(0));
     }
     collide_cell<F, CT, R>(f, omega, omega_minus, [&](int i, R v) {
-        St::store(at<WIDE>(plane_ptr(nxt_f, i, plane), cell), v, kOffsetStorage<ST> ? R(F::w[i]) : R(0));
+        St::template store<NT>(at<WIDE>(plane_ptr(nxt_f, i, plane), cell), v, kOffsetStorage<ST> ? R(F::w[i]) : R(0));
     });
     if constexpr (kOffsetStorage<ST>) {
 #pragma unroll
@@ -61,8 +62,8 @@ __device__ __forceinline__ void reactive_cell(const typename Storage<ST>::S* __r
     collide_scalar<S, R>(gb, m.ux, m.uy, m.uz, omega_c, source);
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
-        St::store(at<WIDE>(plane_ptr(nxt_a, i, plane), scell), ga[i], R(S::w[i]) * ref_a);
-        St::store(at<WIDE>(plane_ptr(nxt_b, i, plane), scell), gb[i], R(S::w[i]) * ref_b);
+        St::template store<NT>(at<WIDE>(plane_ptr(nxt_a, i, plane), scell), ga[i], R(S::w[i]) * ref_a);
+        St::template store<NT>(at<WIDE>(plane_ptr(nxt_b, i, plane), scell), gb[i], R(S::w[i]) * ref_b);
     }
 }
 
@@ -71,7 +72,7 @@ __device__ __forceinline__ void reactive_cell(const typename Storage<ST>::S* __r
 // (lbc_fast.hpp), the velocity taken from the deviations as stored, the scalar
 // collision with 1/cs2 multiplied and the rest equilibrium by remainder, the
 // reaction increment without cancellation (lbc_fast.hpp).
-template <class F, int CT, class S, int ST, bool WIDE = false>
+template <class F, int CT, class S, int ST, bool WIDE = false, bool NT = true>
 __device__ __forceinline__ void reactive_cell_fast(const typename Storage<ST>::S* __restrict__ cur_f,
                                                    typename Storage<ST>::S* __restrict__ nxt_f,
                                                    const typename Storage<ST>::S* __restrict__ cur_a,
@@ -91,8 +92,9 @@ __device__ __forceinline__ void reactive_cell_fast(const typename Storage<ST>::S
         const uint32_t src = pf.src(F::cx[i], F::cy[i], F::cz[i]);
         d[i] = St::load_dev(at<WIDE>(plane_ptr(cur_f, i, plane), src), R(F::w[i]));
     }
-    collide_dev<F, CT, R>(d, omega, omega_minus,
-                          [&](int i, R v) { St::store_dev(at<WIDE>(plane_ptr(nxt_f, i, plane), cell), v, R(F::w[i])); });
+    collide_dev<F, CT, R>(d, omega, omega_minus, [&](int i, R v) {
+        St::template store_dev<NT>(at<WIDE>(plane_ptr(nxt_f, i, plane), cell), v, R(F::w[i]));
+    });
 #pragma unroll
     for (int i = 0; i < F::Q; ++i) d[i] = St::roundtrip_dev(d[i], R(F::w[i]));
     const DevMacro<F, R> m = dev_macro<F, R>(d);
@@ -110,8 +112,8 @@ __device__ __forceinline__ void reactive_cell_fast(const typename Storage<ST>::S
     collide_scalar_fast<S, R>(gb, cb, m.ux, m.uy, m.uz, omega_c, source);
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
-        St::store(at<WIDE>(plane_ptr(nxt_a, i, plane), scell), ga[i], R(S::w[i]) * ref_a);
-        St::store(at<WIDE>(plane_ptr(nxt_b, i, plane), scell), gb[i], R(S::w[i]) * ref_b);
+        St::template store<NT>(at<WIDE>(plane_ptr(nxt_a, i, plane), scell), ga[i], R(S::w[i]) * ref_a);
+        St::template store<NT>(at<WIDE>(plane_ptr(nxt_b, i, plane), scell), gb[i], R(S::w[i]) * ref_b);
     }
 }
 

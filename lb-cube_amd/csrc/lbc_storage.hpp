@@ -17,9 +17,14 @@ namespace lbc {
 template <int ST> struct Storage;
 
 // Every population store is written once and read back only by the next
-// launch, so it is issued as a streaming (non-temporal) store: it does not
-// displace the lines the same launch still reads.
-template <class T> __device__ __forceinline__ void put(T* p, T v) { __builtin_nontemporal_store(v, p); }
+// launch.  NT: a streaming (non-temporal) store, which does not displace the
+// lines the same launch still reads; else an ordinary one, which stays in the
+// caches and lets waves that share a line merge their parts of it.  The
+// launchers choose by size and alignment (streaming_stores, lbc_launch.hpp).
+template <bool NT = true, class T> __device__ __forceinline__ void put(T* p, T v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
 // Population loads stay ordinary cached loads: the x-shifted pulls of one wave
 // share cache lines with its neighbours' loads.  (Non-temporal loads speed up
 // a plain copy by ~5% on MI355X but measured ~1-3% slower here.)
@@ -29,10 +34,10 @@ template <> struct Storage<kF32> {
     using S = float;
     using R = float;
     __device__ static R load(const S* p, R) { return get(p); }
-    __device__ static void store(S* p, R v, R) { put(p, v); }
+    template <bool NT = true> __device__ static void store(S* p, R v, R) { put<NT>(p, v); }
     // deviation form: d = f - w on load, f = w + d on store
     __device__ static R load_dev(const S* p, R w) { return get(p) - w; }
-    __device__ static void store_dev(S* p, R d, R w) { put(p, static_cast<S>(w + d)); }
+    template <bool NT = true> __device__ static void store_dev(S* p, R d, R w) { put<NT>(p, static_cast<S>(w + d)); }
     __device__ static R roundtrip(R v, R) { return v; }
     // the deviation a later load_dev returns after store_dev(d, w)
     __device__ static R roundtrip_dev(R d, R w) { return (w + d) - w; }
@@ -42,9 +47,9 @@ template <> struct Storage<kF64> {
     using S = double;
     using R = double;
     __device__ static R load(const S* p, R) { return get(p); }
-    __device__ static void store(S* p, R v, R) { put(p, v); }
+    template <bool NT = true> __device__ static void store(S* p, R v, R) { put<NT>(p, v); }
     __device__ static R load_dev(const S* p, R w) { return get(p) - w; }
-    __device__ static void store_dev(S* p, R d, R w) { put(p, static_cast<S>(w + d)); }
+    template <bool NT = true> __device__ static void store_dev(S* p, R d, R w) { put<NT>(p, static_cast<S>(w + d)); }
     __device__ static R roundtrip(R v, R) { return v; }
     __device__ static R roundtrip_dev(R d, R w) { return (w + d) - w; }
 };
@@ -53,14 +58,16 @@ template <> struct Storage<kF16> {
     using S = uint16_t;
     using R = float;
     __device__ static R load(const S* p, R off) { return off + static_cast<float>(__builtin_bit_cast(_Float16, get(p))); }
-    __device__ static void store(S* p, R v, R off) {
-        put(p, __builtin_bit_cast(uint16_t, static_cast<_Float16>(v - off)));
+    template <bool NT = true> __device__ static void store(S* p, R v, R off) {
+        put<NT>(p, __builtin_bit_cast(uint16_t, static_cast<_Float16>(v - off)));
     }
     // The value a later load of a stored v returns.
     __device__ static R roundtrip(R v, R off) { return off + static_cast<float>(static_cast<_Float16>(v - off)); }
     // fluid deviations are stored as they are
     __device__ static R load_dev(const S* p, R) { return static_cast<float>(__builtin_bit_cast(_Float16, get(p))); }
-    __device__ static void store_dev(S* p, R d, R) { put(p, __builtin_bit_cast(uint16_t, static_cast<_Float16>(d))); }
+    template <bool NT = true> __device__ static void store_dev(S* p, R d, R) {
+        put<NT>(p, __builtin_bit_cast(uint16_t, static_cast<_Float16>(d)));
+    }
     __device__ static R roundtrip_dev(R d, R) { return static_cast<float>(static_cast<_Float16>(d)); }
 };
 
@@ -76,12 +83,12 @@ template <> struct Storage<kBF16> {
         x += 0x7fffu + ((x >> 16) & 1u);
         return static_cast<uint16_t>(x >> 16);
     }
-    __device__ static void store(S* p, R v, R off) { put(p, encode(v - off)); }
+    template <bool NT = true> __device__ static void store(S* p, R v, R off) { put<NT>(p, encode(v - off)); }
     __device__ static R roundtrip(R v, R off) {
         return off + __builtin_bit_cast(float, static_cast<uint32_t>(encode(v - off)) << 16);
     }
     __device__ static R load_dev(const S* p, R) { return __builtin_bit_cast(float, static_cast<uint32_t>(get(p)) << 16); }
-    __device__ static void store_dev(S* p, R d, R) { put(p, encode(d)); }
+    template <bool NT = true> __device__ static void store_dev(S* p, R d, R) { put<NT>(p, encode(d)); }
     __device__ static R roundtrip_dev(R d, R) {
         return __builtin_bit_cast(float, static_cast<uint32_t>(encode(d)) << 16);
     }
