@@ -715,6 +715,16 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
                                                                   s.block.y, s.block.z, on));
     };
     auto step = [&](St in, St out) { return step_on(st, in, out); };
+    auto seg_len = [&](size_t sgp) { return static_cast<int>(std::min<size_t>(interval, steps - sgp * interval)); };
+    // state t of segment sgp: the checkpoint, or its slot in segment buffer sgp % 2
+    auto state_in = [&](size_t sgp, int t) {
+        return t == 0 ? ckpt + sgp * se : seg + ((sgp & 1) * L.seg_slots + static_cast<size_t>(t)) * se;
+    };
+    // The forward run leaves the states of the last two segments where the
+    // sweep reads them, in the two segment buffers, so those segments are not
+    // run a second time (D3Q19 FP32 at 128^3, four segments of 32: 62 of 124
+    // recomputed steps; 512^2, sixteen of 64: 126 of 1008).
+    auto kept = [&](size_t sgp) { return sgp + 2 >= L.nseg; };
     // forward with checkpoints at the segment starts
     if ((e = hipMemcpyAsync(ckpt, f0, QF * cells * sizeof(R), hipMemcpyDeviceToDevice, st)) != hipSuccess) return e;
     if ((e = hipMemcpyAsync(ckpt + QF * cells, a0, QS * cells * sizeof(R), hipMemcpyDeviceToDevice, st)) !=
@@ -725,11 +735,13 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
         return e;
     R* last = nullptr;
     for (size_t sg = 0; sg < L.nseg; ++sg) {
-        const int len = static_cast<int>(std::min<size_t>(interval, steps - sg * interval));
+        const int len = seg_len(sg);
         St cur(ckpt + sg * se, cells);
         for (int t = 0; t < len; ++t) {
-            const bool to_ckpt = (t == len - 1) && (sg + 1 < L.nseg);
-            R* dst = to_ckpt ? ckpt + (sg + 1) * se : seg + ((t & 1) ? se : 0);
+            R* dst = nullptr;
+            if (t + 1 < len) dst = kept(sg) ? state_in(sg, t + 1) : seg + ((t & 1) ? se : 0);
+            else if (sg + 1 < L.nseg) dst = ckpt + (sg + 1) * se;
+            else dst = seg + (sg & 1) * L.seg_slots * se;  // the final state: slot 0, which no segment's state takes
             St out(dst, cells);
             if ((e = step(cur, out)) != hipSuccess) return e;
             cur = out;
@@ -748,7 +760,7 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     // waits per segment cost more than the overlap gains (with interval 1 the
     // step rose from 24 to 34 us at 512^2).
     constexpr int kOverlapSteps = 8;
-    const bool overlap = interval >= kOverlapSteps && L.nseg > 1;
+    const bool overlap = interval >= kOverlapSteps && L.nseg > 2;
     SweepStreams ss;
     if (overlap) {
         if ((e = ss.create()) != hipSuccess) return e;
@@ -772,26 +784,20 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     // neither kernel fills the GPU.  Events order each walk after its
     // recompute and each recompute after the walk that last read its buffer
     // (without overlap everything runs in order on `stream`).
-    auto seg_len = [&](size_t sgp) { return static_cast<int>(std::min<size_t>(interval, steps - sgp * interval)); };
-    auto state_in = [&](size_t sgp, int t) {
-        return t == 0 ? ckpt + sgp * se : seg + ((sgp & 1) * L.seg_slots + static_cast<size_t>(t)) * se;
-    };
     auto recompute = [&](size_t sgp) {
         hipError_t err = hipSuccess;
         for (int t = 0; t + 1 < seg_len(sgp) && err == hipSuccess; ++t)
             err = step_on(rs, St(state_in(sgp, t), cells), St(state_in(sgp, t + 1), cells));
         return err == hipSuccess && overlap ? hipEventRecord(ss.recomputed[sgp & 1], ss.side) : err;
     };
-    if ((e = recompute(L.nseg - 1)) != hipSuccess) return e;
     for (size_t sgp = L.nseg; sgp-- > 0;) {
         const int len = seg_len(sgp);
-        if (sgp >= 1) {
-            if (overlap && sgp + 1 < L.nseg &&
-                (e = hipStreamWaitEvent(ss.side, ss.swept[(sgp + 1) & 1], 0)) != hipSuccess)
-                return e;
-            if (overlap && (e = recompute(sgp - 1)) != hipSuccess) return e;
+        const bool again = sgp >= 1 && !kept(sgp - 1);  // the previous segment is recomputed
+        if (overlap && again) {
+            if ((e = hipStreamWaitEvent(ss.side, ss.swept[(sgp + 1) & 1], 0)) != hipSuccess) return e;
+            if ((e = recompute(sgp - 1)) != hipSuccess) return e;
         }
-        if (overlap && (e = hipStreamWaitEvent(st, ss.recomputed[sgp & 1], 0)) != hipSuccess) return e;
+        if (overlap && !kept(sgp) && (e = hipStreamWaitEvent(st, ss.recomputed[sgp & 1], 0)) != hipSuccess) return e;
         auto state_at = [&](int t) { return state_in(sgp, t); };
         for (int t = len - 1; t >= 0; --t) {
             St fw(state_at(t), cells);
@@ -809,7 +815,7 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
         }
         if (overlap && (e = hipEventRecord(ss.swept[sgp & 1], st)) != hipSuccess) return e;
         // in order on one stream, the previous segment is recomputed after this walk
-        if (!overlap && sgp >= 1 && (e = recompute(sgp - 1)) != hipSuccess) return e;
+        if (!overlap && again && (e = recompute(sgp - 1)) != hipSuccess) return e;
     }
     // adjoints of the stored initial populations
     StA fin(nu1, cells);
