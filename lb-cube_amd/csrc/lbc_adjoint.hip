@@ -344,8 +344,8 @@ template <class R> __device__ __forceinline__ void mrt27_operator(const R* lam, 
 
 // F, S: the fluid and species lattices; RF: the forward states' type (the
 // trajectory); R: the adjoint's state and arithmetic (R = double with RF =
-// float: the FP64 adjoint of an FP32 run).
-template <class F, class S, class RF, class R, int CT, int MAXT>
+// float: the FP64 adjoint of an FP32 run).  NT: the store form.
+template <class F, class S, class RF, class R, int CT, int MAXT, bool NT>
 __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
     const RF* __restrict__ f, const RF* __restrict__ a, const RF* __restrict__ b, const R* __restrict__ nuf1,
     const R* __restrict__ nua1, const R* __restrict__ nub1, R* __restrict__ nuf0, R* __restrict__ nua0,
@@ -430,8 +430,8 @@ __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
         const R sw = wa + wb;
 #pragma unroll
         for (int j = 0; j < QS; ++j) {
-            put(plane_ptr(nua0, j, plane) + cell, (R(1) - omega_c) * la[j] + omega_c * ea + sw * dsa);
-            put(plane_ptr(nub0, j, plane) + cell, (R(1) - omega_c) * lb[j] + omega_c * eb + sw * dsb);
+            put<NT>(plane_ptr(nua0, j, plane) + cell, (R(1) - omega_c) * la[j] + omega_c * ea + sw * dsa);
+            put<NT>(plane_ptr(nub0, j, plane) + cell, (R(1) - omega_c) * lb[j] + omega_c * eb + sw * dsb);
         }
         const R lux = omega_c * inv_cs2 * (ca * pax + cb * pbx);
         const R luy = omega_c * inv_cs2 * (ca * pay + cb * pby);
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
 #pragma unroll
                 for (int r = 0; r < 19; ++r)
                     if (B.m[r][i] != 0) t += R(B.m[r][i]) * nm[r];
-                put(plane_ptr(nuf0, i, plane) + cell, t + grho + R(F::cx[i]) * gjx + R(F::cy[i]) * gjy +
+                put<NT>(plane_ptr(nuf0, i, plane) + cell, t + grho + R(F::cx[i]) * gjx + R(F::cy[i]) * gjy +
                                                           R(F::cz[i]) * gjz);
             }
         } else if constexpr (CT == kMRT && QF == 27) {
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
             feq_transpose<F, R>(w, m.ux, m.uy, m.uz, al, bx, by, bz);
 #pragma unroll
             for (int i = 0; i < 27; ++i)
-                put(plane_ptr(nuf0, i, plane) + cell, lf[i] - w[i] + al + dev(i, bx, by, bz));
+                put<NT>(plane_ptr(nuf0, i, plane) + cell, lf[i] - w[i] + al + dev(i, bx, by, bz));
         } else if constexpr (CT == kMRT) {
             // f' = M^-1 [(I - S) M f + S m_eq(rho, j)], M^-1 = M^T D^-1
             // (collide_mrt_d2q9): J^T lam = M^T (I - S) mu + (d m_eq/d f)^T S mu
@@ -522,20 +522,20 @@ __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
 #pragma unroll
                 for (int r = 0; r < 9; ++r)
                     if (kD2Q9Basis.m[r][i] != 0) t += R(kD2Q9Basis.m[r][i]) * nm[r];
-                put(plane_ptr(nuf0, i, plane) + cell,
+                put<NT>(plane_ptr(nuf0, i, plane) + cell,
                     t + grho + R(D2Q9::cx[i]) * gjx + R(D2Q9::cy[i]) * gjy);
             }
         } else if constexpr (CT == kRLBM) {
             R out[QF];
             rlbm_transpose<F, R>(fl, lf, m, omega, out);
 #pragma unroll
-            for (int i = 0; i < QF; ++i) put(plane_ptr(nuf0, i, plane) + cell, out[i]);
+            for (int i = 0; i < QF; ++i) put<NT>(plane_ptr(nuf0, i, plane) + cell, out[i]);
         } else if constexpr (CT == kBGK) {
             R al, bx, by, bz;
             feq_transpose<F, R>(lf, m.ux, m.uy, m.uz, al, bx, by, bz);
 #pragma unroll
             for (int i = 0; i < QF; ++i)
-                put(plane_ptr(nuf0, i, plane) + cell, (R(1) - omega) * lf[i] + omega * (al + dev(i, bx, by, bz)));
+                put<NT>(plane_ptr(nuf0, i, plane) + cell, (R(1) - omega) * lf[i] + omega * (al + dev(i, bx, by, bz)));
         } else {
             R lp[QF], lm[QF];
 #pragma unroll
@@ -548,7 +548,7 @@ __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
             feq_transpose<F, R>(lm, m.ux, m.uy, m.uz, am, bxm, bym, bzm);
 #pragma unroll
             for (int i = 0; i < QF; ++i)
-                put(plane_ptr(nuf0, i, plane) + cell, lf[i] - omega * lp[i] - omega_minus * lm[i] +
+                put<NT>(plane_ptr(nuf0, i, plane) + cell, lf[i] - omega * lp[i] - omega_minus * lm[i] +
                                                           omega * (ap + dev(i, bxp, byp, bzp)) +
                                                           omega_minus * (am + dev(i, bxm, bym, bzm)));
         }
@@ -688,8 +688,6 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
                         int interval,
                         double omega_d, double omega_c_d, double k_d, double* J_out, R* gf, R* ga, R* gb,
                         double* djdwc_out, char* ws, hipStream_t st) {
-    LaunchShape sa = s;  // the adjoint's blocks
-    sa.cells.order = F::D == 2 && sizeof(RA) <= 4 ? kContiguousOrder : kDispatchOrder;
     using St = State<F, S, R>;
     using StA = State<F, S, RA>;
     const int storage = std::is_same<R, double>::value ? kF64 : kF32;
@@ -701,6 +699,14 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     RA* nu1 = nu0 + se;
     double* part = reinterpret_cast<double*>(ws + L.off_part);
     double* red = reinterpret_cast<double*>(ws + L.off_red);
+    // The sweep's stores and block order follow plan_traffic on its own two
+    // levels, which stay in the caches where they fit (512^2 FP32, 40 MB:
+    // ordinary stores and ordered blocks 26.0-26.1 ms for 1024 steps, dispatch
+    // order 26.4, streaming 27.4-27.7; 128^3, 554 MB: streaming 40.2 ms for 128
+    // steps, ordinary 40.7-41.2).
+    LaunchShape sa = s;
+    const Traffic sweep = plan_traffic<F::D, RA>(s, address(nu0), cells, 2 * kStatePlanes<F, S> * cells * sizeof(RA));
+    sa.cells.order = sweep.order;
     // the forward's parameters as it rounds them, widened for the adjoint
     const RA omega = static_cast<RA>(static_cast<R>(omega_d)), omega_c = static_cast<RA>(static_cast<R>(omega_c_d));
     const RA k = static_cast<RA>(static_cast<R>(k_d));
@@ -802,14 +808,17 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
         for (int t = len - 1; t >= 0; --t) {
             St fw(state_at(t), cells);
             StA in(nu1, cells), out(nu0, cells);
-            if (s.threads() <= 256)
-                hipLaunchKernelGGL((reactive_adjoint_kernel<F, S, R, RA, CT, 256>), s.grid, s.block, 0, st, fw.f,
-                                   fw.a, fw.b, in.f, in.a, in.b, out.f, out.a, out.b, sa.cells, omega, wm, omega_c, k,
-                                   part);
-            else
-                hipLaunchKernelGGL((reactive_adjoint_kernel<F, S, R, RA, CT, 1024>), s.grid, s.block, 0, st, fw.f,
-                                   fw.a, fw.b, in.f, in.a, in.b, out.f, out.a, out.b, sa.cells, omega, wm, omega_c, k,
-                                   part);
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, s.grid, s.block, 0, st, fw.f, fw.a, fw.b, in.f, in.a, in.b, out.f, out.a,
+                                   out.b, sa.cells, omega, wm, omega_c, k, part);
+            };
+            auto pick = [&](auto maxt) {
+                constexpr int M = decltype(maxt)::value;
+                sweep.streaming ? go(reactive_adjoint_kernel<F, S, R, RA, CT, M, true>)
+                                : go(reactive_adjoint_kernel<F, S, R, RA, CT, M, false>);
+            };
+            if (s.threads() <= 256) pick(std::integral_constant<int, 256>{});
+            else pick(std::integral_constant<int, 1024>{});
             if ((e = hipGetLastError()) != hipSuccess) return e;
             std::swap(nu0, nu1);
         }
