@@ -11,16 +11,16 @@
 // streaming).  One adjoint step per cell:
 //   1. reverse-pull nu_f, nu_a, nu_b of step n+1 (the adjoints of the stored
 //      f_{n+1}, a_{n+1}, b_{n+1} at this cell);
-//   2. pull f_n and take its density and velocity, which the collision
-//      conserves: u' of the forward reaction step up to rounding;
+//   2. take the density and velocity of f_{n+1}, which the collision conserves
+//      and the forward run has left behind (kCompact), or pull f_n for them;
 //   3. reaction step transpose: scalar BGK + source Jacobians, the reaction
 //      Jacobian of the exact one-step map, and the velocity coupling into the
 //      fluid adjoint through du'/df' = (c - u') / rho';
 //   4. fluid collision transpose at the pre-collision state (BGK, TRT with
 //      its even/odd split, MRT through the moment basis, or RLBM through the
 //      non-equilibrium stress it reconstructs from), written to nu_f of step n.
-// Long runs use checkpoints every `interval` steps and recompute each
-// segment forward before walking it backward (lbc_reactive_gradient).
+// Long runs use checkpoints and recompute the segments that the workspace
+// does not hold before walking them backward (lbc_trajectory.hpp).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -32,7 +32,9 @@
 #include "lbc_fast.hpp"
 #include "lbc_launch.hpp"
 #include "lbc_physics.hpp"
+#include "lbc_reactive.hpp"
 #include "lbc_storage.hpp"
+#include "lbc_trajectory.hpp"
 
 namespace lbc {
 
@@ -342,8 +344,48 @@ template <class R> __device__ __forceinline__ void mrt27_operator(const R* lam, 
     for (int i = 0; i < 27; ++i) w[i] = p[g27(L::cx[i] + 1, L::cy[i] + 1, L::cz[i] + 1)];
 }
 
+// What the sweep needs of a forward step is its species and the density and
+// velocity of its fluid; only the regularized collision's transpose also takes
+// the populations.  kCompact: the forward run leaves density and velocity (1 +
+// D planes) in place of the Q populations.  Both runs are bound by memory: the
+// sweep moves 84 planes a step for D3Q19's 99, the forward step 70 for 66, and
+// the workspace holds almost twice the steps (18 planes for 33), which then are
+// not run twice (D3Q19 FP32 at 128^3, 128 steps, interval 32: 40.2 -> 32.6 ms,
+// of which 62 recomputed steps -> 9; D2Q9 FP32 at 512^2, 1024 steps, interval
+// 64: 26.1 -> 24.8 ms).  The FP64 sweep of an FP32 run keeps the populations: it
+// forms density and velocity in FP64.
+template <class RF, class R, int CT> constexpr bool kCompact = CT != kRLBM && std::is_same<RF, R>::value;
+
+// The forward step of the compact trajectory: lbc_reactive_fused_step's cell,
+// which also stores density and velocity (`macro`, 1 + D planes).
+template <class F, int CT, class S, int ST, bool FAST, int MAXT, bool NT>
+__global__ __launch_bounds__(MAXT) void reactive_trace_kernel(
+    const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
+    const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
+    const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b,
+    typename Storage<ST>::S* __restrict__ macro, Cells c, typename Storage<ST>::R omega,
+    typename Storage<ST>::R omega_minus, typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react) {
+    using R = typename Storage<ST>::R;
+    const uint32_t cell = ordered_block(c.order) * blockDim.x + threadIdx.x;
+    if (cell >= c.count) return;
+    const CellCoord q = cell_coord(cell, c);
+    const Pull p(cell, q.x, q.y, q.z, static_cast<int>(c.nx), static_cast<int>(c.ny), static_cast<int>(c.nz));
+    const size_t plane = c.count;
+    Macro<R> m;
+    if constexpr (FAST)
+        m = reactive_cell_fast<F, CT, S, ST, false, NT>(cur_f, nxt_f, cur_a, nxt_a, cur_b, nxt_b, p, p, plane, omega,
+                                                        omega_minus, omega_c, k_react, R(0), R(0));
+    else
+        m = reactive_cell<F, CT, S, ST, false, NT>(cur_f, nxt_f, cur_a, nxt_a, cur_b, nxt_b, p, p, plane, omega,
+                                                   omega_minus, omega_c, k_react, R(0), R(0));
+    put<NT>(at(macro, cell), m.rho);
+    put<NT>(at(plane_ptr(macro, 1, plane), cell), m.ux);
+    put<NT>(at(plane_ptr(macro, 2, plane), cell), m.uy);
+    if constexpr (F::D == 3) put<NT>(at(plane_ptr(macro, 3, plane), cell), m.uz);
+}
+
 // F, S: the fluid and species lattices; RF: the forward states' type (the
-// trajectory); R: the adjoint's state and arithmetic (R = double with RF =
+// trajectory; f: the populations, or kCompact's density and velocity); R: the adjoint's state and arithmetic (R = double with RF =
 // float: the FP64 adjoint of an FP32 run).  NT: the store form.
 template <class F, class S, class RF, class R, int CT, int MAXT, bool NT>
 __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
@@ -366,16 +408,26 @@ __global__ __launch_bounds__(MAXT) void reactive_adjoint_kernel(
         R fl[QF], lf[QF];
 #pragma unroll
         for (int i = 0; i < QF; ++i) {
-            const uint32_t src = pull.src(F::cx[i], F::cy[i], F::cz[i]);
             const uint32_t rev = pull.src(-F::cx[i], -F::cy[i], -F::cz[i]);
-            fl[i] = static_cast<R>(plane_ptr(f, i, plane)[src]);
+            if constexpr (!kCompact<RF, R, CT>) {
+                const uint32_t src = pull.src(F::cx[i], F::cy[i], F::cz[i]);
+                fl[i] = static_cast<R>(plane_ptr(f, i, plane)[src]);
+            }
             lf[i] = plane_ptr(nuf1, i, plane)[rev];
         }
         // BGK, TRT, MRT and RLBM conserve rho and j, so the velocity the forward
         // scalar step read from the post-collision state equals that of the
-        // pulled state up to rounding: the linearisation point is taken from
-        // the pulled populations, without re-colliding them.
-        const Macro<R> m = macro_state<F, R>(fl);
+        // pulled state up to rounding: either serves as the linearisation
+        // point, without re-colliding the populations.
+        Macro<R> m;
+        if constexpr (kCompact<RF, R, CT>) {
+            m.rho = f[cell];
+            m.ux = plane_ptr(f, 1, plane)[cell];
+            m.uy = plane_ptr(f, 2, plane)[cell];
+            m.uz = F::D == 3 ? plane_ptr(f, 3, plane)[cell] : R(0);
+        } else {
+            m = macro_state<F, R>(fl);
+        }
         const Macro<R>& mp = m;
         R ga[QS], gb[QS], la[QS], lb[QS];
 #pragma unroll
@@ -621,8 +673,8 @@ template <class R> __global__ __launch_bounds__(256) void partial_sum_kernel(con
 }
 
 struct GradLayout {
-    size_t cells, state_elems, es, nseg, seg_slots, blocks;
-    size_t off_ckpt, off_seg, off_nu, off_part, off_red, total;
+    size_t capacity, blocks;  // capacity: population planes of the trajectory
+    size_t off_nu, off_part, off_red, total;
 };
 
 constexpr size_t kAlign = 256;
@@ -631,19 +683,14 @@ inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 // planes: population planes of one state (Q of the fluid + 2 Q of the species).
 inline GradLayout grad_layout(size_t es, size_t planes, uint64_t cells, int steps, int interval, dim3 grid) {
     GradLayout L{};
-    L.cells = cells;
-    L.state_elems = planes * L.cells;
-    L.es = es;
-    L.nseg = (static_cast<size_t>(steps) + interval - 1) / interval;
-    L.seg_slots = static_cast<size_t>(interval);
+    const size_t state = planes * cells, nseg = (static_cast<size_t>(steps) + interval - 1) / interval;
+    L.capacity = trajectory_capacity(planes, steps, interval);
     L.blocks = static_cast<size_t>(grid.x) * grid.y;
-    size_t off = 0;
-    L.off_ckpt = off;
-    off = align_up(off + L.nseg * L.state_elems * es);  // states at the segment starts
-    L.off_seg = off;
-    off = align_up(off + 2 * L.seg_slots * L.state_elems * es);  // two recomputed segments
+    // the trajectory, at the workspace's start
+    size_t off = align_up(nseg * state * es);
+    off = align_up(off + 2 * static_cast<size_t>(interval) * state * es);
     L.off_nu = off;
-    off = align_up(off + 2 * L.state_elems * sizeof(double));  // adjoint ping-pong (FP64 or FP32 elements)
+    off = align_up(off + 2 * state * sizeof(double));  // adjoint ping-pong (FP64 or FP32 elements)
     L.off_part = off;
     off = align_up(off + L.blocks * sizeof(double));
     L.off_red = off;
@@ -652,12 +699,15 @@ inline GradLayout grad_layout(size_t es, size_t planes, uint64_t cells, int step
     return L;
 }
 
-// One state of the loop in a workspace slot: the fluid's Q planes, then each
-// species' Q planes.
-template <class F, class S, class R> struct State {
+// One state of the loop: the fluid's Q planes and each species' Q planes.
+template <class R> struct State {
     R *f, *a, *b;
-    State(R* base, size_t cells) : f(base), a(base + F::Q * cells), b(base + (F::Q + S::Q) * cells) {}
 };
+
+// The three in one run of planes.
+template <class F, class S, class R> State<R> packed_state(R* base, size_t cells) {
+    return {base, base + F::Q * cells, base + (F::Q + S::Q) * cells};
+}
 
 // The second stream of the reverse sweep and the events that order it
 // against the caller's stream; destroyed when the sweep ends or fails.
@@ -688,13 +738,19 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
                         int interval,
                         double omega_d, double omega_c_d, double k_d, double* J_out, R* gf, R* ga, R* gb,
                         double* djdwc_out, char* ws, hipStream_t st) {
-    using St = State<F, S, R>;
-    using StA = State<F, S, RA>;
-    const int storage = std::is_same<R, double>::value ? kF64 : kF32;
-    const GradLayout L = grad_layout(sizeof(R), kStatePlanes<F, S>, s.cells.count, steps, interval, s.grid);
-    const size_t cells = L.cells, se = L.state_elems;
-    R* ckpt = reinterpret_cast<R*>(ws + L.off_ckpt);
-    R* seg = reinterpret_cast<R*>(ws + L.off_seg);
+    using St = State<R>;
+    using StA = State<RA>;
+    constexpr bool kTrace = kCompact<R, RA, CT>;
+    constexpr size_t QF = F::Q, QS = S::Q, kMacro = 1 + F::D;
+    constexpr int storage = std::is_same<R, double>::value ? kF64 : kF32;
+    const size_t cells = s.cells.count, se = kStatePlanes<F, S> * cells;
+    const GradLayout L = grad_layout(sizeof(R), kStatePlanes<F, S>, cells, steps, interval, s.grid);
+    const TrajectoryPlanes planes = trajectory_layout(kTrace, F::D, QF, QS);
+    const TrajectoryPlan plan = plan_trajectory(planes, steps, L.capacity);
+    if (plan.length == 0) return hipErrorInvalidValue;
+    R* const ckpt = reinterpret_cast<R*>(ws);  // of the segments but the first
+    R* const slots = ckpt + (plan.segments - 1) * planes.checkpoint * cells;
+    R* const levels = slots + std::min<size_t>(plan.segments, 2) * plan.length * planes.slot * cells;
     RA* nu0 = reinterpret_cast<RA*>(ws + L.off_nu);
     RA* nu1 = nu0 + se;
     double* part = reinterpret_cast<double*>(ws + L.off_part);
@@ -713,52 +769,89 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     const RA wm = CT == kTRT ? static_cast<RA>(trt_omega_minus<R>(static_cast<R>(omega_d))) : RA(0);
     const uint32_t forward_flags = flags & static_cast<uint32_t>(LBC_FLAG_FAST);
     hipError_t e;
-    constexpr size_t QF = F::Q, QS = S::Q;
-    auto step_on = [&](hipStream_t on, St in, St out) {
+    const R fw_omega = static_cast<R>(omega_d), fw_omega_c = static_cast<R>(omega_c_d), fw_k = static_cast<R>(k_d);
+    const R fw_wm = CT == kTRT ? trt_omega_minus<R>(fw_omega) : R(0);
+    // one forward step; `macro`: where its density and velocity go, if anywhere
+    auto step = [&](hipStream_t on, St in, St out, R* macro) {
+        if constexpr (kTrace) {
+            if (macro != nullptr) {
+                LaunchShape sf = s;
+                const Traffic t = adr_traffic<F::D, R>(
+                    sf, false, address(out.f) | address(out.a) | address(out.b) | address(macro), 2 * QF + 4 * QS);
+                const uint32_t lds = capped_residency_adr<F::D, storage, true>() ? capped_lds(s.threads()) : 0;
+                auto go = [&](auto kern) {
+                    hipLaunchKernelGGL(kern, s.grid, s.block, lds, on, in.f, out.f, in.a, out.a, in.b, out.b, macro,
+                                       sf.cells, fw_omega, fw_wm, fw_omega_c, fw_k);
+                };
+                auto form = [&](auto fast, auto maxt) {
+                    constexpr bool FA = decltype(fast)::value;
+                    constexpr int M = decltype(maxt)::value;
+                    t.streaming ? go(reactive_trace_kernel<F, CT, S, storage, FA, M, true>)
+                                : go(reactive_trace_kernel<F, CT, S, storage, FA, M, false>);
+                };
+                auto width = [&](auto fast) {
+                    if (s.threads() <= 256) form(fast, std::integral_constant<int, 256>{});
+                    else form(fast, std::integral_constant<int, 1024>{});
+                };
+                if (forward_flags & LBC_FLAG_FAST) width(std::true_type{});
+                else width(std::false_type{});
+                return hipGetLastError();
+            }
+        }
         return static_cast<hipError_t>(lbc_reactive_fused_step_ex(F::id, CT, S::id, storage, forward_flags, in.f,
                                                                   out.f, in.a, out.a, in.b, out.b, s.nx, s.ny, s.nz,
                                                                   omega_d, omega_c_d, k_d, 0.0, 0.0, s.block.x,
                                                                   s.block.y, s.block.z, on));
     };
-    auto step = [&](St in, St out) { return step_on(st, in, out); };
-    auto seg_len = [&](size_t sgp) { return static_cast<int>(std::min<size_t>(interval, steps - sgp * interval)); };
-    // state t of segment sgp: the checkpoint, or its slot in segment buffer sgp % 2
-    auto state_in = [&](size_t sgp, int t) {
-        return t == 0 ? ckpt + sgp * se : seg + ((sgp & 1) * L.seg_slots + static_cast<size_t>(t)) * se;
+    const size_t nseg = plan.segments;
+    const int first_len = static_cast<int>(plan.first(steps));
+    auto seg_len = [&](size_t sgp) { return sgp == 0 ? first_len : static_cast<int>(plan.length); };
+    // slot t of segment sgp, in segment buffer sgp % 2, and what it holds: the
+    // species and the fluid's populations, or its density and velocity (kTrace)
+    auto slot = [&](size_t sgp, size_t t) {
+        return slots + ((sgp & 1) * plan.length + t) * planes.slot * cells;
     };
-    // The forward run leaves the states of the last two segments where the
-    // sweep reads them, in the two segment buffers, so those segments are not
-    // run a second time (D3Q19 FP32 at 128^3, four segments of 32: 62 of 124
-    // recomputed steps; 512^2, sixteen of 64: 126 of 1008).
-    auto kept = [&](size_t sgp) { return sgp + 2 >= L.nseg; };
-    // forward with checkpoints at the segment starts
-    if ((e = hipMemcpyAsync(ckpt, f0, QF * cells * sizeof(R), hipMemcpyDeviceToDevice, st)) != hipSuccess) return e;
-    if ((e = hipMemcpyAsync(ckpt + QF * cells, a0, QS * cells * sizeof(R), hipMemcpyDeviceToDevice, st)) !=
-        hipSuccess)
-        return e;
-    if ((e = hipMemcpyAsync(ckpt + (QF + QS) * cells, b0, QS * cells * sizeof(R), hipMemcpyDeviceToDevice, st)) !=
-        hipSuccess)
-        return e;
-    R* last = nullptr;
-    for (size_t sg = 0; sg < L.nseg; ++sg) {
+    auto slot_state = [&](size_t sgp, size_t t, R* fluid) {
+        R* const at = slot(sgp, t);
+        if (kTrace) return St{fluid, at + kMacro * cells, at + (kMacro + QS) * cells};
+        return packed_state<F, S>(at, cells);
+    };
+    auto level = [&](int t) { return levels + (t & 1) * QF * cells; };  // the fluid's two levels (kTrace)
+    auto checkpoint = [&](size_t sgp) { return ckpt + (sgp - 1) * planes.checkpoint * cells; };
+    // State t of segment sgp: its start is a checkpoint or the caller's state
+    // (only read), the others are in their slots.
+    auto state_in = [&](size_t sgp, int t) {
+        if (t > 0) return slot_state(sgp, t, level(t));
+        if (sgp == 0) return St{const_cast<R*>(f0), const_cast<R*>(a0), const_cast<R*>(b0)};
+        return packed_state<F, S>(checkpoint(sgp), cells);
+    };
+    // where step t of segment sgp leaves its density and velocity: beside the
+    // checkpoint that it ends in, or in its slot
+    auto macro_of = [&](size_t sgp, int t) {
+        return t + 1 == seg_len(sgp) && sgp + 1 < nseg ? checkpoint(sgp + 1) + se : slot(sgp, t);
+    };
+    // The forward run leaves the last two segments where the sweep reads them.
+    // The others pass through slots 0, whose states nothing else takes, as the
+    // final state does.
+    auto kept = [&](size_t sgp) { return sgp + 2 >= nseg; };
+    St last{};
+    for (size_t sg = 0; sg < nseg; ++sg) {
         const int len = seg_len(sg);
-        St cur(ckpt + sg * se, cells);
+        St cur = state_in(sg, 0);
         for (int t = 0; t < len; ++t) {
-            R* dst = nullptr;
-            if (t + 1 < len) dst = kept(sg) ? state_in(sg, t + 1) : seg + ((t & 1) ? se : 0);
-            else if (sg + 1 < L.nseg) dst = ckpt + (sg + 1) * se;
-            else dst = seg + (sg & 1) * L.seg_slots * se;  // the final state: slot 0, which no segment's state takes
-            St out(dst, cells);
-            if ((e = step(cur, out)) != hipSuccess) return e;
-            cur = out;
-            last = dst;
+            St out;
+            if (t + 1 == len) out = sg + 1 < nseg ? state_in(sg + 1, 0) : slot_state(sg, 0, level(t + 1));
+            else out = kept(sg) ? state_in(sg, t + 1) : slot_state(t & 1, 0, level(t + 1));
+            R* const macro = kTrace && (kept(sg) || t + 1 == len) ? macro_of(sg, t) : nullptr;
+            if ((e = step(st, cur, out, macro)) != hipSuccess) return e;
+            cur = last = out;
         }
     }
     // J = <A>(0) - <A>(T)
     // (fixed-order two-level sums: 512 per-block partials in red[512..1023], then one block)
     hipLaunchKernelGGL((partial_sum_kernel<R>), dim3(512), dim3(256), 0, st, a0, QS * cells, red + 512);
     hipLaunchKernelGGL((sum_kernel<double>), dim3(1), dim3(256), 0, st, red + 512, 512, red);
-    hipLaunchKernelGGL((partial_sum_kernel<R>), dim3(512), dim3(256), 0, st, last + QF * cells, QS * cells,
+    hipLaunchKernelGGL((partial_sum_kernel<R>), dim3(512), dim3(256), 0, st, last.a, QS * cells,
                        red + 512);
     hipLaunchKernelGGL((sum_kernel<double>), dim3(1), dim3(256), 0, st, red + 512, 512, red + 1);
     // The recomputes may overwrite the forward's scratch states from here on.
@@ -766,7 +859,7 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     // waits per segment cost more than the overlap gains (with interval 1 the
     // step rose from 24 to 34 us at 512^2).
     constexpr int kOverlapSteps = 8;
-    const bool overlap = interval >= kOverlapSteps && L.nseg > 2;
+    const bool overlap = plan.length >= kOverlapSteps && nseg > 2;
     SweepStreams ss;
     if (overlap) {
         if ((e = ss.create()) != hipSuccess) return e;
@@ -784,7 +877,7 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     if ((e = hipGetLastError()) != hipSuccess) return e;
     // Reverse sweep.  Segment sgp's states 1..len-1 are recomputed into
     // segment buffer sgp % 2 (slots 1..len-1; state 0 is the checkpoint
-    // itself, and with interval 1 nothing is recomputed) on the side stream,
+    // itself, and segments of one step need nothing) on the side stream,
     // while the caller's stream walks segment sgp + 1 backward from the other
     // buffer: the two are independent, and at a few hundred thousand cells
     // neither kernel fills the GPU.  Events order each walk after its
@@ -793,10 +886,10 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     auto recompute = [&](size_t sgp) {
         hipError_t err = hipSuccess;
         for (int t = 0; t + 1 < seg_len(sgp) && err == hipSuccess; ++t)
-            err = step_on(rs, St(state_in(sgp, t), cells), St(state_in(sgp, t + 1), cells));
+            err = step(rs, state_in(sgp, t), state_in(sgp, t + 1), kTrace ? macro_of(sgp, t) : nullptr);
         return err == hipSuccess && overlap ? hipEventRecord(ss.recomputed[sgp & 1], ss.side) : err;
     };
-    for (size_t sgp = L.nseg; sgp-- > 0;) {
+    for (size_t sgp = nseg; sgp-- > 0;) {
         const int len = seg_len(sgp);
         const bool again = sgp >= 1 && !kept(sgp - 1);  // the previous segment is recomputed
         if (overlap && again) {
@@ -804,10 +897,10 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
             if ((e = recompute(sgp - 1)) != hipSuccess) return e;
         }
         if (overlap && !kept(sgp) && (e = hipStreamWaitEvent(st, ss.recomputed[sgp & 1], 0)) != hipSuccess) return e;
-        auto state_at = [&](int t) { return state_in(sgp, t); };
         for (int t = len - 1; t >= 0; --t) {
-            St fw(state_at(t), cells);
-            StA in(nu1, cells), out(nu0, cells);
+            St fw = state_in(sgp, t);
+            if (kTrace) fw.f = macro_of(sgp, t);
+            const StA in = packed_state<F, S>(nu1, cells), out = packed_state<F, S>(nu0, cells);
             auto go = [&](auto kern) {
                 hipLaunchKernelGGL(kern, s.grid, s.block, 0, st, fw.f, fw.a, fw.b, in.f, in.a, in.b, out.f, out.a,
                                    out.b, sa.cells, omega, wm, omega_c, k, part);
@@ -827,7 +920,7 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
         if (!overlap && again && (e = recompute(sgp - 1)) != hipSuccess) return e;
     }
     // adjoints of the stored initial populations
-    StA fin(nu1, cells);
+    const StA fin = packed_state<F, S>(nu1, cells);
     hipLaunchKernelGGL((reverse_pull_kernel<RA, R, F>), s.grid, s.block, 0, st, fin.f, gf, s.cells, RA(0));
     hipLaunchKernelGGL((reverse_pull_kernel<RA, R, S>), s.grid, s.block, 0, st, fin.a, ga, s.cells, inv_n);
     hipLaunchKernelGGL((reverse_pull_kernel<RA, R, S>), s.grid, s.block, 0, st, fin.b, gb, s.cells, RA(0));

@@ -152,38 +152,6 @@ __global__ __launch_bounds__(MAXT) void reactive_pull_kernel(
     }
 }
 
-// Residency cap (kCappedWavesPerCu, lbc_launch.hpp), measured on the 256^3
-// TGV with two D3Q7 species.  FP32: scalar step 41.2k -> 45.0k MLUPS,
-// reaction step 30.9k -> 31.8k, fused TRT step 21.0k -> 21.3k (both forms).
-// FP16: the fused step gains 3-4.5% (39.2k -> 40.4k, deviation form 39.3k ->
-// 41.1k), the scalar step loses 7%, the reaction step gains 1.4% (left
-// uncapped).  BF16 loses up to 15% and FP64 is unchanged, so both stay
-// uncapped, as do 2D grids (the fused 2048^2 step lost 1-5%).
-template <int D, int ST, bool FUSED> constexpr bool capped_residency_adr() {
-    return D == 3 && (ST == kF32 || (FUSED && ST == kF16));
-}
-
-// The store form and the block order (plan_traffic) of a step whose time loop
-// holds `planes` population planes and that writes at `bases`.  Streaming
-// grids whose loop takes up to kWindowBytes run contiguously (fused step:
-// D2Q9 MRT FP32 at 2048^2, 637 MB, 112 us against 120 in dispatch order and
-// 118 in runs of 8; D3Q19 FP32 at 128^3, 554 MB, 103 against 110 us; fluid and
-// reaction step at 1448^2 FP64 139 against 144 us); above it contiguous runs
-// lose (2048 x 4096 FP32, 1.3 GB, 240 against 232 us; 192^3 FP32 363 against
-// 344 us).  Tiled buffers and planes of more than 4 GiB stream, in dispatch
-// order.
-constexpr uint64_t kWindowBytes = 730ull << 20;
-
-template <int D, class T>
-Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t planes) {
-    const uint64_t footprint = planes * s.cells.count * sizeof(T);
-    Traffic t = plan_traffic<D, T>(s, bases, s.cells.count, footprint);
-    if (t.streaming && footprint <= kWindowBytes) t.order = kContiguousOrder;
-    if (tiled || wide_planes<T>(s)) t = Traffic{true, kDispatchOrder};
-    s.cells.order = t.order;
-    return t;
-}
-
 // Calls go<WIDE, TILED, NT> of the instantiations a launch may take.
 template <class Go> void pick_form(bool wide, bool tiled, bool streaming, Go go) {
     using Y = std::true_type;

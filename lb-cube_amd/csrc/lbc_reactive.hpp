@@ -3,6 +3,7 @@
 #pragma once
 
 #include "lbc_fast.hpp"
+#include "lbc_launch.hpp"
 #include "lbc_physics.hpp"
 #include "lbc_storage.hpp"
 
@@ -19,18 +20,16 @@ namespace lbc {
 // at the same cell (src/simulate_reaction.cpp:527-541); here they are still in
 // registers.  With reduced-precision storage they are passed through the
 // storage rounding first, so the velocity is the one the unfused pair sees.
-// Shared by the single-domain kernel below and the ensemble kernel.
+// Shared by the single-domain, ensemble and gradient kernels.  Returns the
+// density and velocity of the new fluid state.
 template <class F, int CT, class S, int ST, bool WIDE = false, bool NT = true>
-__device__ __forceinline__ void reactive_cell(const typename Storage<ST>::S* __restrict__ cur_f,
-                                              typename Storage<ST>::S* __restrict__ nxt_f,
-                                              const typename Storage<ST>::S* __restrict__ cur_a,
-                                              typename Storage<ST>::S* __restrict__ nxt_a,
-                                              const typename Storage<ST>::S* __restrict__ cur_b,
-                                              typename Storage<ST>::S* __restrict__ nxt_b, const Pull& pf,
-                                              const Pull& ps, size_t plane, typename Storage<ST>::R omega,
-                                              typename Storage<ST>::R omega_minus, typename Storage<ST>::R omega_c,
-                                              typename Storage<ST>::R k_react, typename Storage<ST>::R ref_a,
-                                              typename Storage<ST>::R ref_b) {
+__device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell(
+    const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
+    const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
+    const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b, const Pull& pf,
+    const Pull& ps, size_t plane, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
+    typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react, typename Storage<ST>::R ref_a,
+    typename Storage<ST>::R ref_b) {
     using St = Storage<ST>;
     using R = typename St::R;
     const uint32_t cell = pf.dst, scell = ps.dst;
@@ -65,6 +64,7 @@ __device__ __forceinline__ void reactive_cell(const typename Storage<ST>::S* __r
         St::template store<NT>(at<WIDE>(plane_ptr(nxt_a, i, plane), scell), ga[i], R(S::w[i]) * ref_a);
         St::template store<NT>(at<WIDE>(plane_ptr(nxt_b, i, plane), scell), gb[i], R(S::w[i]) * ref_b);
     }
+    return m;
 }
 
 // The same step in the deviation form (LBC_FLAG_FAST; BGK, TRT, MRT): fluid
@@ -73,16 +73,13 @@ __device__ __forceinline__ void reactive_cell(const typename Storage<ST>::S* __r
 // collision with 1/cs2 multiplied and the rest equilibrium by remainder, the
 // reaction increment without cancellation (lbc_fast.hpp).
 template <class F, int CT, class S, int ST, bool WIDE = false, bool NT = true>
-__device__ __forceinline__ void reactive_cell_fast(const typename Storage<ST>::S* __restrict__ cur_f,
-                                                   typename Storage<ST>::S* __restrict__ nxt_f,
-                                                   const typename Storage<ST>::S* __restrict__ cur_a,
-                                                   typename Storage<ST>::S* __restrict__ nxt_a,
-                                                   const typename Storage<ST>::S* __restrict__ cur_b,
-                                                   typename Storage<ST>::S* __restrict__ nxt_b, const Pull& pf,
-                                                   const Pull& ps, size_t plane, typename Storage<ST>::R omega,
-                                                   typename Storage<ST>::R omega_minus,
-                                                   typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react,
-                                                   typename Storage<ST>::R ref_a, typename Storage<ST>::R ref_b) {
+__device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell_fast(
+    const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
+    const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
+    const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b, const Pull& pf,
+    const Pull& ps, size_t plane, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
+    typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react, typename Storage<ST>::R ref_a,
+    typename Storage<ST>::R ref_b) {
     using St = Storage<ST>;
     using R = typename St::R;
     const uint32_t cell = pf.dst, scell = ps.dst;
@@ -115,6 +112,39 @@ __device__ __forceinline__ void reactive_cell_fast(const typename Storage<ST>::S
         St::template store<NT>(at<WIDE>(plane_ptr(nxt_a, i, plane), scell), ga[i], R(S::w[i]) * ref_a);
         St::template store<NT>(at<WIDE>(plane_ptr(nxt_b, i, plane), scell), gb[i], R(S::w[i]) * ref_b);
     }
+    return Macro<R>{m.rho, m.ux, m.uy, m.uz};
+}
+
+// Residency cap (kCappedWavesPerCu, lbc_launch.hpp), measured on the 256^3
+// TGV with two D3Q7 species.  FP32: scalar step 41.2k -> 45.0k MLUPS,
+// reaction step 30.9k -> 31.8k, fused TRT step 21.0k -> 21.3k (both forms).
+// FP16: the fused step gains 3-4.5% (39.2k -> 40.4k, deviation form 39.3k ->
+// 41.1k), the scalar step loses 7%, the reaction step gains 1.4% (left
+// uncapped).  BF16 loses up to 15% and FP64 is unchanged, so both stay
+// uncapped, as do 2D grids (the fused 2048^2 step lost 1-5%).
+template <int D, int ST, bool FUSED> constexpr bool capped_residency_adr() {
+    return D == 3 && (ST == kF32 || (FUSED && ST == kF16));
+}
+
+// The store form and the block order (plan_traffic) of a step whose time loop
+// holds `planes` population planes and that writes at `bases`.  Streaming
+// grids whose loop takes up to kWindowBytes run contiguously (fused step:
+// D2Q9 MRT FP32 at 2048^2, 637 MB, 112 us against 120 in dispatch order and
+// 118 in runs of 8; D3Q19 FP32 at 128^3, 554 MB, 103 against 110 us; fluid and
+// reaction step at 1448^2 FP64 139 against 144 us); above it contiguous runs
+// lose (2048 x 4096 FP32, 1.3 GB, 240 against 232 us; 192^3 FP32 363 against
+// 344 us).  Tiled buffers and planes of more than 4 GiB stream, in dispatch
+// order.
+constexpr uint64_t kWindowBytes = 730ull << 20;
+
+template <int D, class T>
+Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t planes) {
+    const uint64_t footprint = planes * s.cells.count * sizeof(T);
+    Traffic t = plan_traffic<D, T>(s, bases, s.cells.count, footprint);
+    if (t.streaming && footprint <= kWindowBytes) t.order = kContiguousOrder;
+    if (tiled || wide_planes<T>(s)) t = Traffic{true, kDispatchOrder};
+    s.cells.order = t.order;
+    return t;
 }
 
 }  // namespace lbc
