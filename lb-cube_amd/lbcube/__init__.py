@@ -44,9 +44,9 @@ SCALAR_PAIRS = {("D2Q9", "D2Q5"), ("D3Q19", "D3Q7"), ("D3Q27", "D3Q7")}
 
 
 def _stream(stream):
-    if stream is None:
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return ctypes.c_void_p(stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream))
+    if stream is None:  # torch.cuda.current_stream().cuda_stream without the Stream object
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
 def _extents(lattice, t):
@@ -61,7 +61,8 @@ def _extents(lattice, t):
 def _check_pop(lattice, t, name):
     if not (t.is_cuda and t.is_contiguous()):
         raise ValueError(f"{name} must be a contiguous CUDA tensor")
-    if t.dim() != DIM[lattice] + 1 or t.shape[0] != Q[lattice]:
+    shape = t.shape
+    if len(shape) != DIM[lattice] + 1 or shape[0] != Q[lattice]:
         raise ValueError(f"{name} must have shape (Q={Q[lattice]}, ...) with {DIM[lattice]} spatial axes")
     if t.dtype not in STORAGE:
         raise ValueError(f"{name}: unsupported dtype {t.dtype}")
@@ -73,12 +74,13 @@ def _check_set(named):
     the storage code from one dtype, so a mismatch would read or write past
     the end of a smaller allocation."""
     (n0, t0), rest = named[0], named[1:]
+    cells, dtype, device = t0.shape[1:], t0.dtype, t0.device
     for n, t in rest:
-        if tuple(t.shape[1:]) != tuple(t0.shape[1:]):
-            raise ValueError(f"{n} covers cells {tuple(t.shape[1:])}, {n0} covers {tuple(t0.shape[1:])}")
-        if t.dtype != t0.dtype:
+        if t.shape[1:] != cells:
+            raise ValueError(f"{n} covers cells {tuple(t.shape[1:])}, {n0} covers {tuple(cells)}")
+        if t.dtype is not dtype:
             raise ValueError(f"{n} has dtype {t.dtype}, {n0} has {t0.dtype}: one storage format per call")
-        if t.device != t0.device:
+        if t.device != device:
             raise ValueError(f"{n} is on {t.device}, {n0} on {t0.device}")
 
 
@@ -88,8 +90,13 @@ def default_block(lattice, nx, ny, nz=1):
     return tuple(out)
 
 
+# lbc_default_block's answer for every lattice and domain (the cells are covered
+# linearly, so only the block's size matters).
+DEFAULT_BLOCK = (256, 1, 1)
+
+
 def _block(lattice, block, nx, ny, nz):
-    return default_block(lattice, nx, ny, nz) if block is None else tuple(block)
+    return DEFAULT_BLOCK if block is None else tuple(block)
 
 
 FLAG_FAST = 1
