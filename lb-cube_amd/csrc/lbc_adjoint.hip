@@ -384,6 +384,108 @@ __global__ __launch_bounds__(MAXT) void reactive_trace_kernel(
     if constexpr (F::D == 3) put<NT>(at(plane_ptr(macro, 3, plane), cell), m.uz);
 }
 
+// Two forward steps of the compact trajectory in one launch (2D).  A block runs
+// the first step on a tile of kPairCols x kPairRows cells, one per work-item,
+// into LDS, and the second on the tile without its rim, so the fluid between
+// the two steps never leaves the chip and half the launches go.  A single step
+// of the domains that stay in the caches is a chain of latencies (launch, loads,
+// stores) more than traffic; the rims repeat 1.22 of the first step.  Gradients,
+// single steps -> pairs: FP32 512^2, 1024 steps, 24.85 -> 21.95 ms; 200^2, 400
+// steps, 4.14 -> 3.66; 600^2, 400 steps, 13.0 -> 11.2; FP64 512^2, 200 steps, 8.35
+// -> 7.47.  Tiles of 32 rows: 23.6 for the first (two blocks per CU); the blocks
+// in dispatch order 26.9, in runs of 8 22.9 (neighbouring tiles share lines).
+// The same values as two single steps: the tile holds the populations as the
+// single step stores them.  macro0 with mid_a and mid_b (the trace of the first
+// step) and macro1 may be null: not kept.
+constexpr uint32_t kPairCols = 32, kPairRows = 16;
+
+// Tiles without their rims in a row of the domain, and in all.
+__host__ __device__ inline uint32_t pair_tiles_across(const Cells& c) { return (c.nx + kPairCols - 3) / (kPairCols - 2); }
+inline uint32_t pair_tiles(const Cells& c) {
+    return pair_tiles_across(c) * ((c.ny + kPairRows - 3) / (kPairRows - 2));
+}
+
+template <class S, class T, int N> struct TileTargets {
+    T (*tile)[N];  // the fluid's planes, then each species'
+    uint32_t at;
+    __device__ __forceinline__ T* f(int i) const { return &tile[i][at]; }
+    __device__ __forceinline__ T* a(int i) const { return &tile[9 + i][at]; }
+    __device__ __forceinline__ T* b(int i) const { return &tile[9 + S::Q + i][at]; }
+};
+
+template <class F, class S, class T, int N> struct TileSources {
+    const T (*tile)[N];
+    uint32_t at;
+    template <class L> __device__ __forceinline__ uint32_t from(int i) const {
+        return at - L::cx[i] - L::cy[i] * static_cast<int>(kPairCols);
+    }
+    __device__ __forceinline__ const T* f(int i) const { return &tile[i][from<F>(i)]; }
+    __device__ __forceinline__ const T* a(int i) const { return &tile[9 + i][from<S>(i)]; }
+    __device__ __forceinline__ const T* b(int i) const { return &tile[9 + S::Q + i][from<S>(i)]; }
+};
+
+template <int CT, int ST, bool FAST>
+__global__ __launch_bounds__(kPairCols * kPairRows) void reactive_trace_pair_kernel(
+    const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
+    const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ mid_a,
+    typename Storage<ST>::S* __restrict__ nxt_a, const typename Storage<ST>::S* __restrict__ cur_b,
+    typename Storage<ST>::S* __restrict__ mid_b, typename Storage<ST>::S* __restrict__ nxt_b,
+    typename Storage<ST>::S* __restrict__ macro0, typename Storage<ST>::S* __restrict__ macro1, Cells c,
+    typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus, typename Storage<ST>::R omega_c,
+    typename Storage<ST>::R k_react) {
+    using T = typename Storage<ST>::S;
+    using R = typename Storage<ST>::R;
+    constexpr int N = kPairCols * kPairRows;
+    __shared__ T tile[9 + 2 * D2Q5::Q][N];
+    const size_t plane = c.count;
+    const uint32_t lx = threadIdx.x % kPairCols, ly = threadIdx.x / kPairCols;
+    const uint32_t across = pair_tiles_across(c);
+    const uint32_t block = ordered_block(kContiguousOrder);
+    const uint32_t by = block / across;
+    // the work-item's cell before the periodic wrap, shifted by one: 0 is column -1
+    const uint32_t wx = (block - by * across) * (kPairCols - 2) + lx, wy = by * (kPairRows - 2) + ly;
+    const bool needed = wx <= c.nx + 1 && wy <= c.ny + 1;
+    const bool inner = lx > 0 && lx + 1 < kPairCols && ly > 0 && ly + 1 < kPairRows && wx <= c.nx && wy <= c.ny;
+    const uint32_t x = wx == 0 ? c.nx - 1 : wx == c.nx + 1 ? 0u : wx - 1;
+    const uint32_t y = wy == 0 ? c.ny - 1 : wy == c.ny + 1 ? 0u : wy - 1;
+    const uint32_t cell = y * c.nx + x;
+    auto leave = [&](T* macro, const Macro<R>& m) {
+        put<false>(at(macro, cell), m.rho);
+        put<false>(at(plane_ptr(macro, 1, plane), cell), m.ux);
+        put<false>(at(plane_ptr(macro, 2, plane), cell), m.uy);
+    };
+    if (needed) {
+        const Pull p(cell, static_cast<int>(x), static_cast<int>(y), 0, static_cast<int>(c.nx),
+                     static_cast<int>(c.ny), 1);
+        const CellSources<D2Q9, D2Q5, T, false> in{cur_f, cur_a, cur_b, p, p, plane};
+        const TileTargets<D2Q5, T, N> out{tile, threadIdx.x};
+        Macro<R> m;
+        if constexpr (FAST)
+            m = reactive_update_fast<D2Q9, CT, D2Q5, ST, false>(in, out, omega, omega_minus, omega_c, k_react, R(0),
+                                                                R(0));
+        else
+            m = reactive_update<D2Q9, CT, D2Q5, ST, false>(in, out, omega, omega_minus, omega_c, k_react, R(0), R(0));
+        if (inner && macro0 != nullptr) {
+            leave(macro0, m);
+#pragma unroll
+            for (int i = 0; i < D2Q5::Q; ++i) {
+                put<false>(at(plane_ptr(mid_a, i, plane), cell), *out.a(i));
+                put<false>(at(plane_ptr(mid_b, i, plane), cell), *out.b(i));
+            }
+        }
+    }
+    __syncthreads();
+    if (!inner) return;
+    const TileSources<D2Q9, D2Q5, T, N> in{tile, threadIdx.x};
+    const CellTargets<T, false> out{nxt_f, nxt_a, nxt_b, cell, cell, plane};
+    Macro<R> m;
+    if constexpr (FAST)
+        m = reactive_update_fast<D2Q9, CT, D2Q5, ST, false>(in, out, omega, omega_minus, omega_c, k_react, R(0), R(0));
+    else
+        m = reactive_update<D2Q9, CT, D2Q5, ST, false>(in, out, omega, omega_minus, omega_c, k_react, R(0), R(0));
+    if (macro1 != nullptr) leave(macro1, m);
+}
+
 // F, S: the fluid and species lattices; RF: the forward states' type (the
 // trajectory; f: the populations, or kCompact's density and velocity); R: the adjoint's state and arithmetic (R = double with RF =
 // float: the FP64 adjoint of an FP32 run).  NT: the store form.
@@ -803,6 +905,28 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
                                                                   omega_d, omega_c_d, k_d, 0.0, 0.0, s.block.x,
                                                                   s.block.y, s.block.z, on));
     };
+    // two forward steps in one launch (kPair); mid.f is not written
+    // Not in the reference's order on small domains: its steps are bound by their
+    // arithmetic, which the rims repeat, on too few tiles for 256 CUs (D2Q9 MRT
+    // FP32 at 333^2, 400 steps: 5.65 ms in single steps, 6.0 in pairs; BGK FP64 at
+    // 600^2, 200 steps: 11.1 and 9.9).  Nor past the caches, where the tiles' short
+    // rows leave partial lines (FP32 at 2048^2, 40 steps: 13.2 and 17.2).
+    constexpr bool kPair = kTrace && F::D == 2;
+    constexpr size_t kPairCells = 1u << 18;
+    const bool pairs = kPair && 2 * se * sizeof(R) <= kCachedBytes &&
+                       ((forward_flags & LBC_FLAG_FAST) != 0 || cells >= kPairCells);
+    auto step_pair = [&](hipStream_t on, St in, St mid, St out, R* macro0, R* macro1) {
+        if constexpr (kPair) {
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(pair_tiles(s.cells)), dim3(kPairCols * kPairRows), 0, on, in.f, out.f,
+                                   in.a, mid.a, out.a, in.b, mid.b, out.b, macro0, macro1, s.cells, fw_omega, fw_wm,
+                                   fw_omega_c, fw_k);
+            };
+            forward_flags & LBC_FLAG_FAST ? go(reactive_trace_pair_kernel<CT, storage, true>)
+                                          : go(reactive_trace_pair_kernel<CT, storage, false>);
+        }
+        return hipGetLastError();
+    };
     const size_t nseg = plan.segments;
     const int first_len = static_cast<int>(plan.first(steps));
     auto seg_len = [&](size_t sgp) { return sgp == 0 ? first_len : static_cast<int>(plan.length); };
@@ -817,11 +941,14 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
         return packed_state<F, S>(at, cells);
     };
     auto level = [&](int t) { return levels + (t & 1) * QF * cells; };  // the fluid's two levels (kTrace)
+    // the level that a step from `fluid` writes
+    auto other = [&](const R* fluid) { return fluid == level(0) ? level(1) : level(0); };
     auto checkpoint = [&](size_t sgp) { return ckpt + (sgp - 1) * planes.checkpoint * cells; };
     // State t of segment sgp: its start is a checkpoint or the caller's state
-    // (only read), the others are in their slots.
-    auto state_in = [&](size_t sgp, int t) {
-        if (t > 0) return slot_state(sgp, t, level(t));
+    // (only read), the others are in their slots, with their fluid (kTrace: one
+    // of the levels).
+    auto state_in = [&](size_t sgp, int t, R* fluid) {
+        if (t > 0) return slot_state(sgp, t, fluid);
         if (sgp == 0) return St{const_cast<R*>(f0), const_cast<R*>(a0), const_cast<R*>(b0)};
         return packed_state<F, S>(checkpoint(sgp), cells);
     };
@@ -837,14 +964,23 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     St last{};
     for (size_t sg = 0; sg < nseg; ++sg) {
         const int len = seg_len(sg);
-        St cur = state_in(sg, 0);
-        for (int t = 0; t < len; ++t) {
-            St out;
-            if (t + 1 == len) out = sg + 1 < nseg ? state_in(sg + 1, 0) : slot_state(sg, 0, level(t + 1));
-            else out = kept(sg) ? state_in(sg, t + 1) : slot_state(t & 1, 0, level(t + 1));
-            R* const macro = kTrace && (kept(sg) || t + 1 == len) ? macro_of(sg, t) : nullptr;
-            if ((e = step(st, cur, out, macro)) != hipSuccess) return e;
+        St cur = state_in(sg, 0, nullptr);
+        for (int t = 0; t < len;) {
+            // the state that a step from cur to state u writes, and where step u - 1 leaves its trace
+            auto target = [&](int u) {
+                R* const fluid = other(cur.f);
+                if (u == len) return sg + 1 < nseg ? state_in(sg + 1, 0, nullptr) : slot_state(sg, 0, fluid);
+                if (kept(sg)) return state_in(sg, u, fluid);
+                return slot_state(cur.a == slot_state(0, 0, nullptr).a ? 1 : 0, 0, fluid);
+            };
+            auto trace = [&](int u) { return kTrace && (kept(sg) || u == len) ? macro_of(sg, u - 1) : nullptr; };
+            const int ahead = pairs && t + 2 <= len ? 2 : 1;
+            const St out = target(t + ahead);
+            e = ahead == 2 ? step_pair(st, cur, target(t + 1), out, trace(t + 1), trace(t + 2))
+                           : step(st, cur, out, trace(t + 1));
+            if (e != hipSuccess) return e;
             cur = last = out;
+            t += ahead;
         }
     }
     // J = <A>(0) - <A>(T)
@@ -855,11 +991,17 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
                        red + 512);
     hipLaunchKernelGGL((sum_kernel<double>), dim3(1), dim3(256), 0, st, red + 512, 512, red + 1);
     // The recomputes may overwrite the forward's scratch states from here on.
-    // Segments shorter than kOverlapSteps stay on `stream`: two cross-stream
-    // waits per segment cost more than the overlap gains (with interval 1 the
-    // step rose from 24 to 34 us at 512^2).
+    // On one stream stay segments shorter than kOverlapSteps (two cross-stream
+    // waits each) and states outside the range where it pays: smaller ones end
+    // before the host has launched the other stream's steps (FP32 128^2, 400
+    // steps: 3.39 ms overlapped, 3.34 not; 256^2 3.85 and 4.08), larger ones fill
+    // the GPU or displace each other from the caches (512^2, 1024 steps, 21.95 and
+    // 22.45; 1024^2, 256 steps, 21.6 and 19.0; FP64 600^2, 200 steps, 10.1 and 9.9).
     constexpr int kOverlapSteps = 8;
-    const bool overlap = plan.length >= kOverlapSteps && nseg > 2;
+    constexpr size_t kOverlapMin = 2u << 20, kOverlapMax = 40u << 20;
+    const size_t state_bytes = se * sizeof(R);
+    const bool overlap = plan.length >= kOverlapSteps && nseg > 2 && state_bytes >= kOverlapMin &&
+                         state_bytes <= kOverlapMax;
     SweepStreams ss;
     if (overlap) {
         if ((e = ss.create()) != hipSuccess) return e;
@@ -885,8 +1027,18 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
     // (without overlap everything runs in order on `stream`).
     auto recompute = [&](size_t sgp) {
         hipError_t err = hipSuccess;
-        for (int t = 0; t + 1 < seg_len(sgp) && err == hipSuccess; ++t)
-            err = step(rs, state_in(sgp, t), state_in(sgp, t + 1), kTrace ? macro_of(sgp, t) : nullptr);
+        const int len = seg_len(sgp);
+        St cur = state_in(sgp, 0, nullptr);
+        for (int t = 0; t + 1 < len && err == hipSuccess;) {
+            R* const fluid = other(cur.f);
+            auto trace = [&](int u) { return kTrace ? macro_of(sgp, u - 1) : nullptr; };
+            const int ahead = pairs && t + 2 < len ? 2 : 1;
+            const St out = state_in(sgp, t + ahead, fluid);
+            err = ahead == 2 ? step_pair(rs, cur, state_in(sgp, t + 1, fluid), out, trace(t + 1), trace(t + 2))
+                             : step(rs, cur, out, trace(t + 1));
+            cur = out;
+            t += ahead;
+        }
         return err == hipSuccess && overlap ? hipEventRecord(ss.recomputed[sgp & 1], ss.side) : err;
     };
     for (size_t sgp = nseg; sgp-- > 0;) {
@@ -898,7 +1050,7 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
         }
         if (overlap && !kept(sgp) && (e = hipStreamWaitEvent(st, ss.recomputed[sgp & 1], 0)) != hipSuccess) return e;
         for (int t = len - 1; t >= 0; --t) {
-            St fw = state_in(sgp, t);
+            St fw = state_in(sgp, t, nullptr);
             if (kTrace) fw.f = macro_of(sgp, t);
             const StA in = packed_state<F, S>(nu1, cells), out = packed_state<F, S>(nu0, cells);
             auto go = [&](auto kern) {

@@ -9,11 +9,38 @@
 
 namespace lbc {
 
-// Fluid step + A + B -> C step of one cell: `pf` locates the cell and its
+// Where one cell's populations come from: `pf` locates the cell and its
 // periodic sources in the fluid planes and `ps` in the species planes (the
 // same pull unless the buffers are stored in tiles, whose gaps differ with the
-// lattices' Q), `plane` is the element stride between population planes;
-// WIDE selects 64-bit per-lane addresses (planes of more than 4 GiB), NT the
+// lattices' Q), `plane` is the element stride between population planes; WIDE
+// selects 64-bit per-lane addresses (planes of more than 4 GiB).
+template <class F, class S, class T, bool WIDE> struct CellSources {
+    const T *__restrict__ cf, *__restrict__ ca, *__restrict__ cb;
+    const Pull &pf, &ps;
+    size_t plane;
+    __device__ __forceinline__ const T* f(int i) const {
+        return at<WIDE>(plane_ptr(cf, i, plane), pf.src(F::cx[i], F::cy[i], F::cz[i]));
+    }
+    __device__ __forceinline__ const T* a(int i) const {
+        return at<WIDE>(plane_ptr(ca, i, plane), ps.src(S::cx[i], S::cy[i], S::cz[i]));
+    }
+    __device__ __forceinline__ const T* b(int i) const {
+        return at<WIDE>(plane_ptr(cb, i, plane), ps.src(S::cx[i], S::cy[i], S::cz[i]));
+    }
+};
+
+// Where they go: the cell's element offsets in the fluid and species planes.
+template <class T, bool WIDE> struct CellTargets {
+    T *__restrict__ nf, *__restrict__ na, *__restrict__ nb;
+    uint32_t cell, scell;
+    size_t plane;
+    __device__ __forceinline__ T* f(int i) const { return at<WIDE>(plane_ptr(nf, i, plane), cell); }
+    __device__ __forceinline__ T* a(int i) const { return at<WIDE>(plane_ptr(na, i, plane), scell); }
+    __device__ __forceinline__ T* b(int i) const { return at<WIDE>(plane_ptr(nb, i, plane), scell); }
+};
+
+// Fluid step + A + B -> C step of one cell: populations read through `in` and
+// stored through `out` (CellSources and CellTargets, or a tile in LDS); NT: the
 // store form.
 // The reaction step of the reference reads the fluid populations that the
 // fluid step has just written
@@ -22,25 +49,18 @@ namespace lbc {
 // storage rounding first, so the velocity is the one the unfused pair sees.
 // Shared by the single-domain, ensemble and gradient kernels.  Returns the
 // density and velocity of the new fluid state.
-template <class F, int CT, class S, int ST, bool WIDE = false, bool NT = true>
-__device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell(
-    const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
-    const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
-    const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b, const Pull& pf,
-    const Pull& ps, size_t plane, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
+template <class F, int CT, class S, int ST, bool NT, class In, class Out>
+__device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_update(
+    const In& in, const Out& out, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
     typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react, typename Storage<ST>::R ref_a,
     typename Storage<ST>::R ref_b) {
     using St = Storage<ST>;
     using R = typename St::R;
-    const uint32_t cell = pf.dst, scell = ps.dst;
     R f[F::Q];
 #pragma unroll
-    for (int i = 0; i < F::Q; ++i) {
-        const uint32_t src = pf.src(F::cx[i], F::cy[i], F::cz[i]);
-        f[i] = St::load(at<WIDE>(plane_ptr(cur_f, i, plane), src), kOffsetStorage<ST> ? R(F::w[i]) : R(0));
-    }
+    for (int i = 0; i < F::Q; ++i) f[i] = St::load(in.f(i), kOffsetStorage<ST> ? R(F::w[i]) : R(0));
     collide_cell<F, CT, R>(f, omega, omega_minus, [&](int i, R v) {
-        St::template store<NT>(at<WIDE>(plane_ptr(nxt_f, i, plane), cell), v, kOffsetStorage<ST> ? R(F::w[i]) : R(0));
+        St::template store<NT>(out.f(i), v, kOffsetStorage<ST> ? R(F::w[i]) : R(0));
     });
     if constexpr (kOffsetStorage<ST>) {
 #pragma unroll
@@ -50,9 +70,8 @@ __device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell(
     R ga[S::Q], gb[S::Q];
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
-        const uint32_t src = ps.src(S::cx[i], S::cy[i], S::cz[i]);
-        ga[i] = St::load(at<WIDE>(plane_ptr(cur_a, i, plane), src), R(S::w[i]) * ref_a);
-        gb[i] = St::load(at<WIDE>(plane_ptr(cur_b, i, plane), src), R(S::w[i]) * ref_b);
+        ga[i] = St::load(in.a(i), R(S::w[i]) * ref_a);
+        gb[i] = St::load(in.b(i), R(S::w[i]) * ref_b);
     }
     const R ca = concentration<S, R>(ga);
     const R cb = concentration<S, R>(gb);
@@ -61,8 +80,8 @@ __device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell(
     collide_scalar<S, R>(gb, m.ux, m.uy, m.uz, omega_c, source);
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
-        St::template store<NT>(at<WIDE>(plane_ptr(nxt_a, i, plane), scell), ga[i], R(S::w[i]) * ref_a);
-        St::template store<NT>(at<WIDE>(plane_ptr(nxt_b, i, plane), scell), gb[i], R(S::w[i]) * ref_b);
+        St::template store<NT>(out.a(i), ga[i], R(S::w[i]) * ref_a);
+        St::template store<NT>(out.b(i), gb[i], R(S::w[i]) * ref_b);
     }
     return m;
 }
@@ -72,35 +91,26 @@ __device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell(
 // (lbc_fast.hpp), the velocity taken from the deviations as stored, the scalar
 // collision with 1/cs2 multiplied and the rest equilibrium by remainder, the
 // reaction increment without cancellation (lbc_fast.hpp).
-template <class F, int CT, class S, int ST, bool WIDE = false, bool NT = true>
-__device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell_fast(
-    const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
-    const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
-    const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b, const Pull& pf,
-    const Pull& ps, size_t plane, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
+template <class F, int CT, class S, int ST, bool NT, class In, class Out>
+__device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_update_fast(
+    const In& in, const Out& out, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
     typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react, typename Storage<ST>::R ref_a,
     typename Storage<ST>::R ref_b) {
     using St = Storage<ST>;
     using R = typename St::R;
-    const uint32_t cell = pf.dst, scell = ps.dst;
     R d[F::Q];
 #pragma unroll
-    for (int i = 0; i < F::Q; ++i) {
-        const uint32_t src = pf.src(F::cx[i], F::cy[i], F::cz[i]);
-        d[i] = St::load_dev(at<WIDE>(plane_ptr(cur_f, i, plane), src), R(F::w[i]));
-    }
-    collide_dev<F, CT, R>(d, omega, omega_minus, [&](int i, R v) {
-        St::template store_dev<NT>(at<WIDE>(plane_ptr(nxt_f, i, plane), cell), v, R(F::w[i]));
-    });
+    for (int i = 0; i < F::Q; ++i) d[i] = St::load_dev(in.f(i), R(F::w[i]));
+    collide_dev<F, CT, R>(d, omega, omega_minus,
+                          [&](int i, R v) { St::template store_dev<NT>(out.f(i), v, R(F::w[i])); });
 #pragma unroll
     for (int i = 0; i < F::Q; ++i) d[i] = St::roundtrip_dev(d[i], R(F::w[i]));
     const DevMacro<F, R> m = dev_macro<F, R>(d);
     R ga[S::Q], gb[S::Q];
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
-        const uint32_t src = ps.src(S::cx[i], S::cy[i], S::cz[i]);
-        ga[i] = St::load(at<WIDE>(plane_ptr(cur_a, i, plane), src), R(S::w[i]) * ref_a);
-        gb[i] = St::load(at<WIDE>(plane_ptr(cur_b, i, plane), src), R(S::w[i]) * ref_b);
+        ga[i] = St::load(in.a(i), R(S::w[i]) * ref_a);
+        gb[i] = St::load(in.b(i), R(S::w[i]) * ref_b);
     }
     const R ca = concentration<S, R>(ga);
     const R cb = concentration<S, R>(gb);
@@ -109,10 +119,38 @@ __device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell_fast(
     collide_scalar_fast<S, R>(gb, cb, m.ux, m.uy, m.uz, omega_c, source);
 #pragma unroll
     for (int i = 0; i < S::Q; ++i) {
-        St::template store<NT>(at<WIDE>(plane_ptr(nxt_a, i, plane), scell), ga[i], R(S::w[i]) * ref_a);
-        St::template store<NT>(at<WIDE>(plane_ptr(nxt_b, i, plane), scell), gb[i], R(S::w[i]) * ref_b);
+        St::template store<NT>(out.a(i), ga[i], R(S::w[i]) * ref_a);
+        St::template store<NT>(out.b(i), gb[i], R(S::w[i]) * ref_b);
     }
     return Macro<R>{m.rho, m.ux, m.uy, m.uz};
+}
+
+template <class F, int CT, class S, int ST, bool WIDE = false, bool NT = true>
+__device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell(
+    const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
+    const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
+    const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b, const Pull& pf,
+    const Pull& ps, size_t plane, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
+    typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react, typename Storage<ST>::R ref_a,
+    typename Storage<ST>::R ref_b) {
+    using T = typename Storage<ST>::S;
+    return reactive_update<F, CT, S, ST, NT>(CellSources<F, S, T, WIDE>{cur_f, cur_a, cur_b, pf, ps, plane},
+                                CellTargets<T, WIDE>{nxt_f, nxt_a, nxt_b, pf.dst, ps.dst, plane}, omega,
+                                omega_minus, omega_c, k_react, ref_a, ref_b);
+}
+
+template <class F, int CT, class S, int ST, bool WIDE = false, bool NT = true>
+__device__ __forceinline__ Macro<typename Storage<ST>::R> reactive_cell_fast(
+    const typename Storage<ST>::S* __restrict__ cur_f, typename Storage<ST>::S* __restrict__ nxt_f,
+    const typename Storage<ST>::S* __restrict__ cur_a, typename Storage<ST>::S* __restrict__ nxt_a,
+    const typename Storage<ST>::S* __restrict__ cur_b, typename Storage<ST>::S* __restrict__ nxt_b, const Pull& pf,
+    const Pull& ps, size_t plane, typename Storage<ST>::R omega, typename Storage<ST>::R omega_minus,
+    typename Storage<ST>::R omega_c, typename Storage<ST>::R k_react, typename Storage<ST>::R ref_a,
+    typename Storage<ST>::R ref_b) {
+    using T = typename Storage<ST>::S;
+    return reactive_update_fast<F, CT, S, ST, NT>(CellSources<F, S, T, WIDE>{cur_f, cur_a, cur_b, pf, ps, plane},
+                                     CellTargets<T, WIDE>{nxt_f, nxt_a, nxt_b, pf.dst, ps.dst, plane}, omega,
+                                     omega_minus, omega_c, k_react, ref_a, ref_b);
 }
 
 // Residency cap (kCappedWavesPerCu, lbc_launch.hpp), measured on the 256^3

@@ -58,3 +58,48 @@ def test_gradient_does_not_depend_on_the_segments(gpu, lattice, shape, collision
         assert got[0] == want[0] and got[4] == want[4], interval
         assert all(torch.equal(x, y) for x, y in zip(got[1:4], want[1:4])), interval
     assert all(torch.equal(x, y) for x, y in zip((f, a, b), keep))
+
+
+# Small domains run the deviation form two steps to a launch, in tiles of 30 x
+# 14 cells, and the reference's order in single steps.  In FP64 the two forms round apart by about 1e-14 of the largest
+# gradient over these steps; a population taken from a wrong cell is off by
+# more than 1e-4 of it.
+EDGES = [(1, 1), (2, 3), (13, 29), (14, 30), (15, 31), (28, 60), (29, 61), (1, 95), (43, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("collision", ["BGK", "TRT", "MRT"])
+@pytest.mark.parametrize("shape,steps", [(s, n) for s in EDGES for n in (2, 5)])
+def test_paired_steps_equal_single_steps(gpu, collision, shape, steps):
+    print(f"case pairs {collision} {shape} steps {steps}", flush=True)
+    f, a, b = state("D2Q9", shape, "f64", gpu)
+    single, pairs = (adjoint.reactive_gradient(collision, f, a, b, steps, 1.6, 1.25, 0.05, 2, fast=fast)
+                     for fast in (False, True))
+    want = adjoint.loss_of(collision, f, a, b, steps, 1.6, 1.25, 0.05, fast=True)
+    assert abs(pairs[0] - want) <= 1e-13 and abs(single[0] - want) <= 1e-13
+    for x, y in zip(pairs[1:4], single[1:4]):
+        assert (x - y).abs().max().item() <= 1e-11 * y.abs().max().item()
+    assert abs(pairs[4] - single[4]) <= 1e-11 * max(abs(single[4]), 1e-3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fast", [False, True])
+def test_paired_gradient_does_not_depend_on_the_segments(gpu, fast):
+    print(f"case paired segments fast={fast}", flush=True)
+    f, a, b = state("D2Q9", (512, 515), "f32", gpu)
+    want, got = (adjoint.reactive_gradient("TRT", f, a, b, 23, 1.6, 1.25, 0.05, iv, fast=fast) for iv in (23, 3))
+    assert got[0] == want[0] and got[4] == want[4]
+    assert all(torch.equal(x, y) for x, y in zip(got[1:4], want[1:4]))
+
+
+# From 2^18 cells on the reference's order also runs in pairs; the FP64 sweep of
+# an FP32 run steps singly.  Their final states, so their losses, are the same.
+@pytest.mark.gpu
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("collision", ["BGK", "TRT", "MRT"])
+def test_paired_loss_equals_single_steps_at_2_18_cells(gpu, collision, fast):
+    print(f"case paired loss {collision} fast={fast}", flush=True)
+    f, a, b = state("D2Q9", (512, 515), "f32", gpu)
+    pairs, single = (adjoint.reactive_gradient(collision, f, a, b, 7, 1.6, 1.25, 0.05, 7, fast=fast, adjoint_f64=w)
+                     for w in (False, True))
+    assert pairs[0] == single[0]
