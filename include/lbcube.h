@@ -297,18 +297,21 @@ int lbc_reactive_fused_step_ex(int fluid_lattice, int collision, int scalar_latt
  * A + B -> C; `steps` calls of lbc_reactive_fused_step from f0, a0, b0) by the
  * discrete adjoint.  loss = <C>(T) = <A>(0) - <A>(T) (domain means).  Outputs:
  * *loss, the adjoints dloss/d(f0, a0, b0) of the initial populations (same
- * layout and type as the inputs) and dloss/d(omega_c).  States are
- * checkpointed every `interval` steps and each segment is recomputed before
- * it is walked backward; the recompute of a segment runs on a private stream
- * of the library (default priority, created and destroyed by the call) while
- * `stream` walks the following segment, ordered by events.  storage: LBC_F32
+ * layout and type as the inputs) and dloss/d(omega_c).  `interval` sizes the
+ * workspace: a state for each `interval` steps and two segments of `interval`
+ * states.  The run is cut into the longest segments that it holds; the last
+ * two stay from the forward run, the others are recomputed from checkpoints
+ * before they are walked backward.  For states of 2 to 40 MB the recompute of a
+ * segment runs on a private stream of the library (default priority, created
+ * and destroyed by the call) while `stream` walks the following segment,
+ * ordered by events.  The gradient does not depend on `interval`.  storage: LBC_F32
  * or LBC_F64.  flags: 0 (forward =
  * lbc_reactive_fused_step) or LBC_FLAG_FAST (forward =
  * lbc_reactive_fused_step_ex(..., LBC_FLAG_FAST, ...)); the adjoint sweep is
  * the same for both; with LBC_F32, LBC_FLAG_F64_ADJOINT carries the adjoint
  * in FP64 on the FP32 trajectory.  The caller passes a
  * device workspace of at least lbc_reactive_gradient_workspace() bytes
- * (checkpoints plus two segment buffers); no device memory is allocated.  block_x * block_y must be a multiple of 64 (whole
+ * and reads f0, a0 and b0 until it returns; no device memory is allocated.  block_x * block_y must be a multiple of 64 (whole
  * wavefronts), else hipErrorInvalidConfiguration.  Synchronizes `stream`.
  * No counterpart in the reference. */
 int lbc_reactive_gradient_workspace(int storage, uint64_t nx, uint64_t ny, int steps, int interval,
@@ -324,8 +327,7 @@ int lbc_reactive_gradient(int collision, int storage, uint32_t flags, const void
  * LBC_D3Q19 / LBC_D3Q27; BGK, TRT, MRT or RLBM, else hipErrorInvalidValue) plus two D3Q7
  * species, `steps` calls of lbc_reactive_fused_step(fluid_lattice,
  * collision, LBC_D3Q7, ...) from f0, a0, b0; loss <A>(0) - <A>(T).  The
- * workspace holds the checkpoints and two segment buffers of states of
- * Q + 14 planes.  Flags, storage, checkpoints, streams, block rule and
+ * workspace is sized as there, in states of Q + 14 planes.  Flags, storage, checkpoints, streams, block rule and
  * synchronisation as lbc_reactive_gradient.  No counterpart in the reference. */
 int lbc_reactive_gradient_workspace_3d(int fluid_lattice, int storage, uint64_t nx, uint64_t ny, uint64_t nz,
                                        int steps, int interval, uint32_t block_x, uint32_t block_y, uint32_t block_z,

@@ -20,7 +20,7 @@ template <int ST> struct Storage;
 // launch.  NT: a streaming (non-temporal) store, which does not displace the
 // lines the same launch still reads; else an ordinary one, which stays in the
 // caches and lets waves that share a line merge their parts of it.  The
-// launchers choose by size and alignment (streaming_stores, lbc_launch.hpp).
+// launchers choose by size and alignment (plan_traffic, lbc_launch.hpp).
 template <bool NT = true, class T> __device__ __forceinline__ void put(T* p, T v) {
     if constexpr (NT) __builtin_nontemporal_store(v, p);
     else *p = v;

@@ -4,8 +4,8 @@ The loop is D2Q9 + two D2Q5 species, or D3Q19 / D3Q27 + two D3Q7 species (BGK,
 TRT, MRT or RLBM), with A + B -> C, stepped by
 lbc_reactive_fused_step; the loss is the domain-mean product <C>(T) =
 <A>(0) - <A>(T).  `reactive_gradient` calls lbc_reactive_gradient (2D) or
-lbc_reactive_gradient_3d (forward with checkpoints every `interval` steps,
-segment recompute, adjoint sweep);
+lbc_reactive_gradient_3d (forward with checkpoints, segment recompute, adjoint
+sweep, in a workspace that `interval` sizes);
 `ReactiveLoss` wraps it as a torch.autograd.Function of the initial
 populations and the scalar relaxation time tau_s, so gradients with respect to
 anything the initial state is built from (for instance a velocity perturbation
