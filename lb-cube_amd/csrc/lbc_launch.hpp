@@ -310,11 +310,23 @@ constexpr uint64_t kCachedBytes = 256ull << 20;
 //    446 us: each XCD's separate window of the 38 streams costs more than the
 //    edge lines save), the other formats in runs of 8 (D3Q19 FP16 at 256^3 223
 //    -> 212 us, BF16 at 256 x 256 x 200 193 -> 185 us, FP64 at 128^3 127 -> 118
-//    us, at 192^3 level).
+//    us, at 192^3 level), but for planes in step (kPlanesInStep).
 //
 // bases: the addresses of the buffers written, ORed; footprint: the bytes of
 // the buffers the step reads and writes.
 constexpr uint64_t kContiguousBytes = 350ull << 20;
+
+// Planes a multiple of 256 MiB apart: the streams of one cell share their
+// channels and cache sets, and in runs eight windows of them meet (D3Q19, each
+// time in four placements of the buffers, runs of 8 against dispatch order: TRT
+// FP16 at 512^3 1.86-2.27 against 1.81-1.92 ms, at 256 x 1024 x 512 1.93-2.06
+// against 1.76-1.87, at 512 x 512 x 1024 4.45 against 3.85; MRT BF16 at 512^3
+// 2.04-2.16 against 1.80-1.94; D3Q27 TRT FP16 2.69-3.10 against 2.61-2.82; FP64
+// at 512 x 512 x 128 2.01-2.09 against 1.93-1.98).  Planes of 128 MiB go both
+// ways by their shape (256 x 256 x 1024 FP16 0.90 against 0.92-0.98 ms, 1024 x
+// 256 x 256 0.90-0.98 against 0.92-0.97), as do FP64 planes of 512 MiB (512 x
+// 512 x 256 3.46-4.03 against 3.57-4.01).
+constexpr uint64_t kPlanesInStep = 256ull << 20;
 
 template <int D, class S>
 Traffic plan_traffic(const LaunchShape& s, uint64_t bases, uint64_t plane, uint64_t footprint) {
@@ -323,7 +335,9 @@ Traffic plan_traffic(const LaunchShape& s, uint64_t bases, uint64_t plane, uint6
     if (!cached && misaligned == 0) {
         if (D == 2 && footprint <= kContiguousBytes) return Traffic{true, kContiguousOrder};
         if (D == 2) return Traffic{true, sizeof(S) <= 4 ? 3u : kDispatchOrder};
-        return Traffic{true, sizeof(S) == 4 ? kDispatchOrder : 3u};
+        const uint64_t bytes = plane * sizeof(S);
+        const bool in_step = bytes % kPlanesInStep == 0 && (sizeof(S) == 2 || bytes == kPlanesInStep);
+        return Traffic{true, sizeof(S) == 4 || in_step ? kDispatchOrder : 3u};
     }
     return Traffic{false, D == 2 && footprint <= kContiguousBytes ? kContiguousOrder : 5u};
 }

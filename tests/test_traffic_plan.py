@@ -1,0 +1,45 @@
+"""Which store form and block order the steps take (the headers' own rules on
+the host): the lines that the measurements beside the rules draw, from both
+sides.  What the forms compute is the same; tests/test_traffic.py compares
+them on the GPU."""
+from __future__ import annotations
+
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+BYTES = {"f64": 8, "f32": 4, "f16": 2}
+DISPATCH, RUNS_OF_8, RUNS_OF_32, CONTIGUOUS = 0, 3, 5, 31
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("traffic") / "traffic_plan_check"
+    subprocess.run(["/opt/rocm/bin/hipcc", "-O1", "-std=c++23", "--offload-arch=gfx950", "-x", "hip",
+                    os.path.join(HERE, "traffic_plan_check.cpp"), "-o", str(exe)], check=True, capture_output=True,
+                   timeout=300)
+
+    def run(cases):
+        """(streaming, order) of each (step, storage, (nx, ny, nz), Q, offset)."""
+        text = "".join(f"{step} {BYTES[st]} {e[0]} {e[1]} {e[2]} {q} {off}\n" for step, st, e, q, off in cases)
+        r = subprocess.run([str(exe)], input=text, capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stdout + r.stderr
+        out = [tuple(int(v) for v in line.split()) for line in r.stdout.splitlines()]
+        assert len(out) == len(cases)
+        return [(bool(s), o) for s, o in out]
+
+    return run
+
+
+def test_planes_a_multiple_of_256_mib_apart_keep_the_dispatch_order(plans):
+    apart = [("f16", (512, 512, 512)), ("f16", (1024, 1024, 128)), ("f16", (512, 512, 1024)), ("f64", (512, 512, 128))]
+    others = [("f16", (256, 256, 256)), ("f16", (512, 512, 480)), ("f16", (512, 512, 256)), ("f16", (640, 640, 640)),
+              ("f64", (256, 256, 256)), ("f64", (512, 512, 256))]
+    cases = [("fluid", st, e, q, 0) for q in (19, 27) for st, e in apart]
+    assert plans(cases) == [(True, DISPATCH)] * len(cases)
+    cases = [("fluid", st, e, q, 0) for q in (19, 27) for st, e in others]
+    assert plans(cases) == [(True, RUNS_OF_8)] * len(cases)
+    cases = [("fluid", "f32", e, 19, 0) for e in ((512, 512, 512), (256, 256, 256), (192, 192, 192))]
+    assert plans(cases) == [(True, DISPATCH)] * len(cases)
