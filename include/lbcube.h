@@ -301,10 +301,11 @@ int lbc_reactive_fused_step_ex(int fluid_lattice, int collision, int scalar_latt
  * workspace: a state for each `interval` steps and two segments of `interval`
  * states.  The run is cut into the longest segments that it holds; the last
  * two stay from the forward run, the others are recomputed from checkpoints
- * before they are walked backward.  For states of 2 to 40 MB the recompute of a
- * segment runs on a private stream of the library (default priority, created
- * and destroyed by the call) while `stream` walks the following segment,
- * ordered by events.  The gradient does not depend on `interval`.  storage: LBC_F32
+ * before they are walked backward.  The recompute of a segment may run on a
+ * private stream of the library (default priority, created and destroyed by
+ * the call) while `stream` walks the following segment, ordered by events: by
+ * the sizes of the state and of the segments, from three segments on.  The
+ * gradient does not depend on `interval`.  storage: LBC_F32
  * or LBC_F64.  flags: 0 (forward =
  * lbc_reactive_fused_step) or LBC_FLAG_FAST (forward =
  * lbc_reactive_fused_step_ex(..., LBC_FLAG_FAST, ...)); the adjoint sweep is

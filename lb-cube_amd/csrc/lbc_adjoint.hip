@@ -991,17 +991,7 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
                        red + 512);
     hipLaunchKernelGGL((sum_kernel<double>), dim3(1), dim3(256), 0, st, red + 512, 512, red + 1);
     // The recomputes may overwrite the forward's scratch states from here on.
-    // On one stream stay segments shorter than kOverlapSteps (two cross-stream
-    // waits each) and states outside the range where it pays: smaller ones end
-    // before the host has launched the other stream's steps (FP32 128^2, 400
-    // steps: 3.39 ms overlapped, 3.34 not; 256^2 3.85 and 4.08), larger ones fill
-    // the GPU or displace each other from the caches (512^2, 1024 steps, 21.95 and
-    // 22.45; 1024^2, 256 steps, 21.6 and 19.0; FP64 600^2, 200 steps, 10.1 and 9.9).
-    constexpr int kOverlapSteps = 8;
-    constexpr size_t kOverlapMin = 2u << 20, kOverlapMax = 40u << 20;
-    const size_t state_bytes = se * sizeof(R);
-    const bool overlap = plan.length >= kOverlapSteps && nseg > 2 && state_bytes >= kOverlapMin &&
-                         state_bytes <= kOverlapMax;
+    const bool overlap = overlapped(plan, se * sizeof(R), F::D, sizeof(R), pairs);
     SweepStreams ss;
     if (overlap) {
         if ((e = ss.create()) != hipSuccess) return e;

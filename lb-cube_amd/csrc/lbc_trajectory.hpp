@@ -44,6 +44,32 @@ inline std::size_t trajectory_capacity(std::size_t state, std::size_t steps, std
     return ((steps + interval - 1) / interval + 2 * interval) * state;
 }
 
+// Whether a segment is recomputed on a second stream while the caller's walks
+// the next one: from three segments on (the last two are never recomputed) of
+// at least kOverlapSteps steps (two cross-stream waits each), for states up to
+// kOverlapMax: larger ones fill the GPU or displace each other from the caches
+// (FP32 D2Q9 512^2, 1024 steps, 21.95 ms overlapped, 22.45 not; 1024^2, 256
+// steps, 21.6 and 19.0; FP64 600^2, 200 steps, 10.6 and 10.4).  Down to the
+// smallest states it pays, where the sweep's launches leave the GPU idle (BGK
+// FP32 400 steps, interval 16, paired: 8^2 3.13 and 3.25 ms, 96^2 3.57 and 3.97,
+// 200^2 3.67 and 4.22; RLBM FP64 1024 steps, interval 32: 64^2 12.4 and 15.1;
+// D3Q19 RLBM FP32 300 steps: 16^3 3.95 and 5.0), except that the host cannot
+// feed two streams with steps shorter than a launch: single 2D steps of FP32
+// states below kShortState32 (FP64: kShortState64) need segments of
+// kShortSteps (RLBM FP32 400 steps, interval 16: 128^2 5.15 and 4.53, 200^2 4.92
+// and 4.91, 240^2 4.75 and 5.17; interval 32, 1024 steps: 128^2 12.1 and 13.0;
+// FP64, interval 16: 16^2 5.01 and 4.71, 24^2 5.03 and 5.33).
+constexpr std::size_t kOverlapSteps = 8, kShortSteps = 32, kOverlapMax = 40u << 20;
+constexpr std::size_t kShortState32 = 4u << 20, kShortState64 = 64u << 10;
+
+// state_bytes: of one state of `element`-byte populations; paired: two steps
+// per launch.
+inline bool overlapped(const TrajectoryPlan& plan, std::size_t state_bytes, std::size_t dim, std::size_t element,
+                       bool paired) {
+    const bool brief = dim == 2 && !paired && state_bytes < (element == 4 ? kShortState32 : kShortState64);
+    return plan.segments > 2 && plan.length >= (brief ? kShortSteps : kOverlapSteps) && state_bytes <= kOverlapMax;
+}
+
 // The planes of a run.  compact: a slot holds the density and velocity of the
 // step's fluid (1 + dim planes) and the species it starts from; two fluid
 // levels beside the slots; a checkpoint also carries the density and velocity
