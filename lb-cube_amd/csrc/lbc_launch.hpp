@@ -298,14 +298,15 @@ constexpr uint64_t kCachedBytes = 256ull << 20;
 //
 // The order, by what was measured (256-work-item blocks):
 //  - ordinary stores, 3D: runs of 32 (runs of 8 to 64 are within 2%).
-//  - ordinary stores, 2D, cache-resident: contiguous (D2Q9 FP64 at 512^2 9.2
-//    us in dispatch order, 7.1 us; FP32 at 1001 x 701 10.3 -> 9.0 us); larger
-//    2D grids runs of 32 (FP32 at 4095 x 2047 120 -> 109 us, contiguous 120).
-//  - streaming stores, 2D: contiguous up to kContiguousBytes (FP32 at 2048^2,
-//    302 MB, 62.6 us in dispatch order, 61.0 in runs of 8, 55.0 contiguous; FP64
-//    at 1448^2 58.4 -> 54.0 us), above it runs of 8 up to 4 bytes per element
-//    (FP32 at 4096 x 2048 107 us in dispatch order, 111 contiguous, 102 in
-//    runs) and FP64 in dispatch order (206 us, 210 in runs).
+//  - 2D up to kContiguousBytes: contiguous, with either store (in the caches
+//    D2Q9 FP64 at 512^2 9.2 us in dispatch order, 7.1 us; FP32 at 1001 x 701 10.3
+//    -> 9.0 us; past them FP32 at 2048^2, 288 MiB, 62.6 us in dispatch order,
+//    61.0 in runs of 8, 55.0 contiguous; FP64 at 1448^2 58.4 -> 54.0 us).
+//  - ordinary stores, larger 2D: runs of 32 (FP32 at 4095 x 2047 120 -> 109 us,
+//    contiguous 120).
+//  - streaming stores, larger 2D: runs of 8 up to 4 bytes per element (FP32 at
+//    4096 x 2048 107 us in dispatch order, 111 contiguous, 102 in runs) and FP64
+//    in dispatch order (206 us, 210 in runs).
 //  - streaming stores, 3D: FP32 in dispatch order (256^3 425 us, in runs of 8
 //    446 us: each XCD's separate window of the 38 streams costs more than the
 //    edge lines save), the other formats in runs of 8 (D3Q19 FP16 at 256^3 223
@@ -313,8 +314,15 @@ constexpr uint64_t kCachedBytes = 256ull << 20;
 //    us, at 192^3 level), but for planes in step (kPlanesInStep).
 //
 // bases: the addresses of the buffers written, ORed; footprint: the bytes of
-// the buffers the step reads and writes.
-constexpr uint64_t kContiguousBytes = 350ull << 20;
+// the buffers that the step's time loop reads and writes.
+//
+// kContiguousBytes: the memory-side cache and the eight L2s of 4 MiB hold 288
+// MiB, and the measured line lies just above: contiguous still wins at 295 MiB
+// (FP64 at 2093 x 1026 56 us, in runs of 32 59-62), loses a little at 297 (FP32
+// at 2048 x 2112 56.6 us, in runs of 8 55.2) and much at 340 (FP32 at 2048 x 2304
+// 71.9 and 60.7; FP64 at 1536^2 70.1, in dispatch order 61.6; FP16 at 3072^2 72.0
+// and 60.2; ordinary stores, FP32 at 2201 x 2199 84.8, in runs of 32 67.4).
+constexpr uint64_t kContiguousBytes = 296ull << 20;
 
 // Planes a multiple of 256 MiB apart: the streams of one cell share their
 // channels and cache sets, and in runs eight windows of them meet (D3Q19, each
@@ -328,18 +336,21 @@ constexpr uint64_t kContiguousBytes = 350ull << 20;
 // 512 x 256 3.46-4.03 against 3.57-4.01).
 constexpr uint64_t kPlanesInStep = 256ull << 20;
 
+// The order past the caches, of planes `plane` elements apart.
+template <int D, class S> uint32_t large_order(bool streaming, uint64_t plane) {
+    if (!streaming) return 5u;
+    if (D == 2) return sizeof(S) <= 4 ? 3u : kDispatchOrder;
+    const uint64_t bytes = plane * sizeof(S);
+    const bool in_step = bytes % kPlanesInStep == 0 && (sizeof(S) == 2 || bytes == kPlanesInStep);
+    return sizeof(S) == 4 || in_step ? kDispatchOrder : 3u;
+}
+
 template <int D, class S>
 Traffic plan_traffic(const LaunchShape& s, uint64_t bases, uint64_t plane, uint64_t footprint) {
     const uint64_t misaligned = (bases | plane * sizeof(S) | static_cast<uint64_t>(s.cells.zgap) * sizeof(S)) % 64;
-    const bool cached = footprint <= kCachedBytes;
-    if (!cached && misaligned == 0) {
-        if (D == 2 && footprint <= kContiguousBytes) return Traffic{true, kContiguousOrder};
-        if (D == 2) return Traffic{true, sizeof(S) <= 4 ? 3u : kDispatchOrder};
-        const uint64_t bytes = plane * sizeof(S);
-        const bool in_step = bytes % kPlanesInStep == 0 && (sizeof(S) == 2 || bytes == kPlanesInStep);
-        return Traffic{true, sizeof(S) == 4 || in_step ? kDispatchOrder : 3u};
-    }
-    return Traffic{false, D == 2 && footprint <= kContiguousBytes ? kContiguousOrder : 5u};
+    const bool streaming = footprint > kCachedBytes && misaligned == 0;
+    if (D == 2 && footprint <= kContiguousBytes) return Traffic{streaming, kContiguousOrder};
+    return Traffic{streaming, large_order<D, S>(streaming, plane)};
 }
 
 }  // namespace lbc

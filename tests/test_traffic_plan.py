@@ -43,3 +43,14 @@ def test_planes_a_multiple_of_256_mib_apart_keep_the_dispatch_order(plans):
     assert plans(cases) == [(True, RUNS_OF_8)] * len(cases)
     cases = [("fluid", "f32", e, 19, 0) for e in ((512, 512, 512), (256, 256, 256), (192, 192, 192))]
     assert plans(cases) == [(True, DISPATCH)] * len(cases)
+
+
+def test_2d_grids_run_contiguously_while_the_caches_hold_their_levels(plans):
+    within = [("f32", (512, 512), 0, False), ("f32", (2048, 2048), 0, True), ("f32", (2048, 2048), 4, False),
+              ("f16", (2880, 2880), 0, True), ("f64", (2048, 1024), 0, True), ("f64", (2093, 1026), 0, False)]
+    got = plans([("fluid", st, e + (1,), 9, off) for st, e, off, _ in within])
+    assert got == [(streaming, CONTIGUOUS) for *_, streaming in within]
+    past = [("f32", (2048, 2112), 0, (True, RUNS_OF_8)), ("f32", (2048, 2304), 0, (True, RUNS_OF_8)),
+            ("f64", (1536, 1536), 0, (True, DISPATCH)), ("f16", (3072, 3072), 0, (True, RUNS_OF_8)),
+            ("f32", (2201, 2199), 0, (False, RUNS_OF_32)), ("f64", (1536, 1536), 8, (False, RUNS_OF_32))]
+    assert plans([("fluid", st, e + (1,), 9, off) for st, e, off, _ in past]) == [want for *_, want in past]
