@@ -164,23 +164,65 @@ template <int D, int ST, bool FUSED> constexpr bool capped_residency_adr() {
     return D == 3 && (ST == kF32 || (FUSED && ST == kF16));
 }
 
-// The store form and the block order (plan_traffic) of a step whose time loop
-// holds `planes` population planes and that writes at `bases`.  Streaming
-// grids whose loop takes up to kWindowBytes run contiguously (fused step:
-// D2Q9 MRT FP32 at 2048^2, 637 MB, 112 us against 120 in dispatch order and
-// 118 in runs of 8; D3Q19 FP32 at 128^3, 554 MB, 103 against 110 us; fluid and
-// reaction step at 1448^2 FP64 139 against 144 us); above it contiguous runs
-// lose (2048 x 4096 FP32, 1.3 GB, 240 against 232 us; 192^3 FP32 363 against
-// 344 us).  Tiled buffers and planes of more than 4 GiB stream, in dispatch
-// order.
-constexpr uint64_t kWindowBytes = 730ull << 20;
+// The memory-side cache has 16 ways of 16 MiB.  Where a small multiple of the
+// plane (q of them) is a multiple of 16 MiB, every q-th plane falls on the same
+// sets; from planes / q > 16 streams on they crowd the ways, and a grid whose
+// blocks all work on one window of each plane loses what the cache held.  A
+// contiguous run per XCD spreads each plane over eight windows.  The least such
+// q up to 4, or 0.
+inline uint64_t crowding(uint64_t plane_bytes, uint64_t planes) {
+    constexpr uint64_t kWay = 16ull << 20, kNear = kWay / 64;
+    for (uint64_t q = 1; q <= 4 && planes > 16 * q; ++q) {
+        const uint64_t end = q * plane_bytes + kNear;
+        if (end >= kWay && end % kWay <= 2 * kNear) return q;
+    }
+    return 0;
+}
 
-template <int D, class T>
-Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t planes) {
-    const uint64_t footprint = planes * s.cells.count * sizeof(T);
-    Traffic t = plan_traffic<D, T>(s, bases, s.cells.count, footprint);
-    if (t.streaming && footprint <= kWindowBytes) t.order = kContiguousOrder;
-    if (tiled || wide_planes<T>(s)) t = Traffic{true, kDispatchOrder};
+// The store form and the block order of a step whose time loop holds `fluid`
+// and `species` population planes and that writes at `bases`.  FUSED: fluid
+// and species in one launch, else the launch of the species alone.  Loops in
+// the caches follow plan_traffic, tiled buffers and planes of more than 4 GiB
+// stream in dispatch order.  Past the caches the general order holds
+// (large_order), but crowded planes run contiguously up to kCrowdedBytes (us,
+// three placements of the buffers or more, general order -> contiguous):
+//  - fused, crowded: D2Q9 MRT FP32 2048^2 109-140 -> 107-118; FP64 2048 x 1024
+//    122-130 -> 109-114; FP16 4096 x 2048 118-124 -> 113-122; D3Q19 TRT FP32 128^3
+//    99-111 -> 94-104, 112^3 69-79 -> 64-70.
+//  - fused, not crowded: 1920^2 FP32 104 -> 125, 3072^2 FP16 135 -> 153, FP64
+//    1152^2 74 -> 82; D3Q19 FP32 120^3 85 -> 94, 136^3 119.5 -> 130, FP16 168^3 123
+//    -> 149; D3Q27 FP32 120^3 106 -> 117.
+//  - crowded past the limit: 2048 x 4096 FP32 229 -> 241; D3Q19 FP16 192 x 256 x
+//    128 161 -> 170, FP32 256 x 128 x 128 195-198 -> 194-204.
+//  - 3D at 2 bytes, where q < 3 gains nothing and the runs lose: in dispatch order
+//    (TRT FP16 256 x 256 x 64 100 us, contiguous 101, runs of 8 103; BF16 512 x 128 x
+//    64 108, 109 and 114).
+constexpr uint64_t kCrowdedBytes = 730ull << 20;
+
+// The launch of the species alone reads what the fluid's launch has left.  2D:
+// in the fluid's order while that is contiguous (D2Q9 and two species, FP64 at
+// 1472^2, loop of two launches: both contiguous 143.6 us, both in dispatch
+// order 139.7, one of each 148.8).  3D: contiguous where crowded up to
+// kCrowdedSpecies (D3Q19 FP32 256 x 128 x 128 247-257 -> 239-247, FP64 128^3
+// 253-275 -> 242-253).
+constexpr uint64_t kCrowdedSpecies = 1100ull << 20;
+
+template <int D, class T, bool FUSED>
+Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t fluid, uint64_t species) {
+    const uint64_t plane = s.cells.count, bytes = plane * sizeof(T), loop = (fluid + species) * bytes;
+    Traffic t = plan_traffic<D, T>(s, bases, plane, loop);
+    if (tiled || wide_planes<T>(s)) {
+        t = Traffic{true, kDispatchOrder};
+    } else if (loop > kCachedBytes) {
+        const uint64_t q = crowding(bytes, fluid + species);
+        const bool crowded = q != 0 && loop <= (FUSED || D == 2 ? kCrowdedBytes : kCrowdedSpecies);
+        t.order = large_order<D, T>(t.streaming, plane);
+        if (crowded && (D == 2 || t.streaming))
+            t.order = D == 3 && sizeof(T) == 2 && q < 3 ? kDispatchOrder : kContiguousOrder;
+        if (!FUSED && D == 2) {
+            if (t.streaming && fluid * bytes <= kContiguousBytes) t.order = kContiguousOrder;
+        }
+    }
     s.cells.order = t.order;
     return t;
 }

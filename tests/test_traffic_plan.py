@@ -54,3 +54,37 @@ def test_2d_grids_run_contiguously_while_the_caches_hold_their_levels(plans):
             ("f64", (1536, 1536), 0, (True, DISPATCH)), ("f16", (3072, 3072), 0, (True, RUNS_OF_8)),
             ("f32", (2201, 2199), 0, (False, RUNS_OF_32)), ("f64", (1536, 1536), 8, (False, RUNS_OF_32))]
     assert plans([("fluid", st, e + (1,), 9, off) for st, e, off, _ in past]) == [want for *_, want in past]
+
+
+def test_fused_steps_run_contiguously_only_where_their_planes_crowd_the_cache_sets(plans):
+    crowded = [("f32", (2048, 2048, 1)), ("f64", (2048, 1024, 1)), ("f16", (4096, 2048, 1)), ("f16", (2880, 2880, 1)),
+               ("f32", (128, 128, 128)), ("f32", (256, 256, 32)), ("f32", (112, 112, 112)), ("f64", (112, 112, 112)),
+               ("f64", (256, 64, 64)), ("f16", (128, 128, 128)), ("f16", (112, 112, 224))]
+    cases = [("fused", st, e, 9 if e[2] == 1 else 19, 0) for st, e in crowded]
+    assert plans(cases) == [(True, CONTIGUOUS)] * len(cases)
+    spread = [("f32", (1920, 1920, 1), (True, RUNS_OF_8)), ("f32", (2048, 2304, 1), (True, RUNS_OF_8)),
+              ("f16", (3072, 3072, 1), (True, RUNS_OF_8)), ("f64", (1152, 1152, 1), (True, DISPATCH)),
+              ("f32", (120, 120, 120), (True, DISPATCH)), ("f32", (136, 136, 136), (True, DISPATCH)),
+              ("f16", (168, 168, 168), (True, RUNS_OF_8)), ("f64", (104, 104, 104), (True, RUNS_OF_8)),
+              # crowded, but past the limit, or at two bytes in one or two groups
+              ("f32", (2048, 4096, 1), (True, RUNS_OF_8)), ("f32", (256, 128, 128), (True, DISPATCH)),
+              ("f16", (192, 256, 128), (True, RUNS_OF_8)), ("f16", (256, 256, 64), (True, DISPATCH))]
+    assert plans([("fused", st, e, 9 if e[2] == 1 else 19, 0) for st, e, _ in spread]) == [want for *_, want in spread]
+    cached = [("f32", (512, 512, 1)), ("f32", (1001, 701, 1)), ("f64", (64, 64, 64)), ("f32", (96, 96, 96))]
+    got = plans([("fused", st, e, 9 if e[2] == 1 else 19, 0) for st, e in cached])
+    assert got == [(False, CONTIGUOUS)] * 2 + [(False, RUNS_OF_32)] * 2
+    # misaligned planes keep ordinary stores
+    got = plans([("fused", "f32", e, 9 if e[2] == 1 else 19, 0)
+                 for e in ((2049, 2047, 1), (1501, 1501, 1), (2501, 2499, 1), (129, 129, 129))])
+    assert got == [(False, CONTIGUOUS)] + [(False, RUNS_OF_32)] * 3
+
+
+def test_species_steps_follow_the_fluids_order_in_2d(plans):
+    for step in ("reaction", "scalar"):
+        cases = [("f32", (1920, 1920, 1), CONTIGUOUS), ("f32", (2048, 2048, 1), CONTIGUOUS),
+                 ("f32", (2048, 2304, 1), RUNS_OF_8), ("f64", (1472, 1472, 1), DISPATCH),
+                 ("f16", (3072, 3072, 1), RUNS_OF_8)]
+        assert plans([(step, st, e, 9, 0) for st, e, _ in cases]) == [(True, order) for *_, order in cases], step
+        assert plans([("fluid", st, e, 9, 0) for st, e, _ in cases[1:]]) == [(True, order) for *_, order in cases[1:]]
+        assert plans([(step, "f32", (128, 128, 128), 19, 0), (step, "f32", (256, 128, 128), 19, 0)]) == \
+            [(True, CONTIGUOUS)] * 2

@@ -1,16 +1,21 @@
 // Host check of the steps' store form and block order (the rules of
-// lb-cube_amd/csrc/lbc_launch.hpp, the headers' own code).  Each line of stdin
-// is "<step> <element bytes> <nx> <ny> <nz> <Q> <offset>": the planes of a
-// domain lie back to back, `offset` bytes past a cache line (nz = 1: 2D).
+// lb-cube_amd/csrc/lbc_launch.hpp and lbc_reactive.hpp, the headers' own code).
+// Each line of stdin is "<step> <element bytes> <nx> <ny> <nz> <Q> <offset>":
+// step is fluid, fused, reaction or scalar, Q the fluid's; the planes of a domain
+// lie back to back, `offset` bytes past a cache line (nz = 1: 2D).
 // Prints "<streaming> <order>" for each.
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 
 #include "../lb-cube_amd/csrc/lbc_launch.hpp"
+#include "../lb-cube_amd/csrc/lbc_reactive.hpp"
 
 template <int D, class T> lbc::Traffic plan(const char* step, lbc::LaunchShape& s, int q, uint64_t base) {
-    (void)step;
+    const uint64_t qs = D == 2 ? 5 : 7;
+    if (std::strcmp(step, "fused") == 0) return lbc::adr_traffic<D, T, true>(s, false, base, 2 * q, 4 * qs);
+    if (std::strcmp(step, "reaction") == 0) return lbc::adr_traffic<D, T, false>(s, false, base, 2 * q, 4 * qs);
+    if (std::strcmp(step, "scalar") == 0) return lbc::adr_traffic<D, T, false>(s, false, base, 2 * q, 2 * qs);
     return lbc::plan_traffic<D, T>(s, base, s.cells.count, 2ull * q * s.cells.count * sizeof(T));
 }
 
