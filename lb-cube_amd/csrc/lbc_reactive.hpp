@@ -204,8 +204,12 @@ constexpr uint64_t kCrowdedBytes = 730ull << 20;
 // 1472^2, loop of two launches: both contiguous 143.6 us, both in dispatch
 // order 139.7, one of each 148.8).  3D: contiguous where crowded up to
 // kCrowdedSpecies (D3Q19 FP32 256 x 128 x 128 247-257 -> 239-247, FP64 128^3
-// 253-275 -> 242-253).
-constexpr uint64_t kCrowdedSpecies = 1100ull << 20;
+// 253-275 -> 242-253).  Else FP64 in runs up to kSpeciesRuns (120^3 214.8 ->
+// 210.5) and in dispatch order above (256^3 2028-2046, in runs of 8 2081-2098;
+// 256 x 256 x 192 1578 and 1681), 2-byte storage in dispatch order (FP16 320^3
+// 1004-1018, in runs 1058-1075, with two scalars 1215 and 1271; from 144^3 to
+// 416^3 else within 2% either way).
+constexpr uint64_t kCrowdedSpecies = 1100ull << 20, kSpeciesRuns = 730ull << 20;
 
 template <int D, class T, bool FUSED>
 Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t fluid, uint64_t species) {
@@ -222,6 +226,8 @@ Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t fluid, 
         if (!FUSED && D == 2) {
             if (t.streaming && fluid * bytes <= kContiguousBytes) t.order = kContiguousOrder;
         }
+        if (!FUSED && D == 3 && t.streaming && !crowded && (sizeof(T) == 2 || (sizeof(T) == 8 && loop > kSpeciesRuns)))
+            t.order = kDispatchOrder;
     }
     s.cells.order = t.order;
     return t;

@@ -88,3 +88,11 @@ def test_species_steps_follow_the_fluids_order_in_2d(plans):
         assert plans([("fluid", st, e, 9, 0) for st, e, _ in cases[1:]]) == [(True, order) for *_, order in cases[1:]]
         assert plans([(step, "f32", (128, 128, 128), 19, 0), (step, "f32", (256, 128, 128), 19, 0)]) == \
             [(True, CONTIGUOUS)] * 2
+
+
+def test_3d_species_steps_in_dispatch_order(plans):
+    for step in ("reaction", "scalar"):
+        cases = [("f64", (256, 256, 256), DISPATCH), ("f64", (256, 256, 192), DISPATCH), ("f64", (104, 104, 104), RUNS_OF_8),
+                 ("f16", (320, 320, 320), DISPATCH), ("f16", (168, 168, 168), DISPATCH), ("f32", (192, 192, 192), DISPATCH),
+                 ("f64", (128, 128, 128), CONTIGUOUS)]
+        assert plans([(step, st, e, 19, 0) for st, e, _ in cases]) == [(True, order) for *_, order in cases], step
