@@ -878,7 +878,7 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
         if constexpr (kTrace) {
             if (macro != nullptr) {
                 LaunchShape sf = s;
-                const Traffic t = adr_traffic<F::D, R, true>(
+                const Traffic t = adr_traffic<F::D, R, kFusedStep>(
                     sf, false, address(out.f) | address(out.a) | address(out.b) | address(macro), 2 * QF, 4 * QS);
                 const uint32_t lds = capped_residency_adr<F::D, storage, true>() ? capped_lds(s.threads()) : 0;
                 auto go = [&](auto kern) {

@@ -172,8 +172,8 @@ hipError_t launch_scalar(const void* ca, void* na, const void* cb, void* nb, con
     const bool tiled = s.cells.zgap != 0 && (S::D == 3 || s.cells.tiles > 1);
     const uint32_t plane = tiled ? s.cells.zgap / (F::Q - 1) : s.cells.count;
     const uint32_t zgap_s = tiled ? (S::Q - 1) * plane : 0u;
-    const Traffic t = adr_traffic<S::D, T, false>(s, tiled, address(na) | (REACT ? address(nb) : 0), 2 * F::Q,
-                                                  (REACT ? 4 : 2) * S::Q);
+    const Traffic t = adr_traffic<S::D, T, REACT ? kReactionStep : kScalarStep>(
+        s, tiled, address(na) | (REACT ? address(nb) : 0), 2 * F::Q, (REACT ? 4 : 2) * S::Q);
     const uint32_t lds = capped_residency_adr<S::D, ST, false>() ? capped_lds(s.threads()) : 0;
     auto args = [&](auto kern) {
         hipLaunchKernelGGL(kern, s.grid, s.block, lds, stream, static_cast<const T*>(ca), static_cast<T*>(na),
@@ -231,7 +231,7 @@ hipError_t launch_fused(const void* cf, void* nf, const void* ca, void* na, cons
     const R w = static_cast<R>(omega);
     const R wm = CT == kTRT ? trt_omega_minus<R>(w) : R(0);
     const Traffic t =
-        adr_traffic<F::D, T, true>(s, tiled, address(nf) | address(na) | address(nb), 2 * F::Q, 4 * S::Q);
+        adr_traffic<F::D, T, kFusedStep>(s, tiled, address(nf) | address(na) | address(nb), 2 * F::Q, 4 * S::Q);
     const uint32_t lds = capped_residency_adr<F::D, ST, true>() ? capped_lds(s.threads()) : 0;
     auto args = [&](auto kern) {
         hipLaunchKernelGGL(kern, s.grid, s.block, lds, stream, static_cast<const T*>(cf), static_cast<T*>(nf),
@@ -284,7 +284,7 @@ hipError_t launch_reactive_pull(const void* cf, void* nf, const void* ca, void* 
     const uint32_t plane = tiled ? s.cells.zgap / (F::Q - 1) : s.cells.count;
     const uint32_t zgap_s = tiled ? (S::Q - 1) * plane : 0u;
     const Traffic t =
-        adr_traffic<F::D, T, true>(s, tiled, address(nf) | address(na) | address(nb), 2 * F::Q, 4 * S::Q);
+        adr_traffic<F::D, T, kFusedStep>(s, tiled, address(nf) | address(na) | address(nb), 2 * F::Q, 4 * S::Q);
     const uint32_t lds = capped_residency_adr<F::D, ST, true>() ? capped_lds(s.threads()) : 0;
     auto args = [&](auto kern) {
         hipLaunchKernelGGL(kern, s.grid, s.block, lds, stream, static_cast<const T*>(cf), static_cast<T*>(nf),

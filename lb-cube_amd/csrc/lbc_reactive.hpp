@@ -180,12 +180,11 @@ inline uint64_t crowding(uint64_t plane_bytes, uint64_t planes) {
 }
 
 // The store form and the block order of a step whose time loop holds `fluid`
-// and `species` population planes and that writes at `bases`.  FUSED: fluid
-// and species in one launch, else the launch of the species alone.  Loops in
-// the caches follow plan_traffic, tiled buffers and planes of more than 4 GiB
-// stream in dispatch order.  Past the caches the general order holds
-// (large_order), but crowded planes run contiguously up to kCrowdedBytes (us,
-// three placements of the buffers or more, general order -> contiguous):
+// and `species` population planes and that writes at `bases`.  Loops in the
+// caches follow plan_traffic, tiled buffers and planes of more than 4 GiB stream
+// in dispatch order.  Past the caches the general order holds (large_order), but
+// crowded planes run contiguously up to kCrowdedBytes (us, three placements of
+// the buffers or more, general order -> contiguous):
 //  - fused, crowded: D2Q9 MRT FP32 2048^2 109-140 -> 107-118; FP64 2048 x 1024
 //    122-130 -> 109-114; FP16 4096 x 2048 118-124 -> 113-122; D3Q19 TRT FP32 128^3
 //    99-111 -> 94-104, 112^3 69-79 -> 64-70.
@@ -209,24 +208,41 @@ constexpr uint64_t kCrowdedBytes = 730ull << 20;
 // 256 x 256 x 192 1578 and 1681), 2-byte storage in dispatch order (FP16 320^3
 // 1004-1018, in runs 1058-1075, with two scalars 1215 and 1271; from 144^3 to
 // 416^3 else within 2% either way).
+// Misaligned 2D planes: streaming stores leave the fluid in the caches.
+// Contiguous up to kSpeciesStream (ordinary -> streaming: two scalars FP32 1801
+// x 1799 120 -> 115, FP64 1301 x 1299 129 -> 121; reaction FP64 1201 x 1199 107 ->
+// 97) and, one species at a time, where crowded (two scalars FP32 2049 x 2047
+// 185 -> 165, FP64 1449 x 1447 178 -> 157; the reaction step FP32 2049 x 2047 157
+// with ordinary stores, 161 streaming), then FP64 scalars in dispatch order up
+// to kSpeciesStream64 (1501 x 1499 181 -> 173, 1551 x 1549 194 -> 185; not the
+// reaction step: 1301 x 1299 118 -> 123, nor FP32 and FP16: 2401 x 2399 240 -> 248,
+// 3001 x 2999 189 -> 195).
 constexpr uint64_t kCrowdedSpecies = 1100ull << 20, kSpeciesRuns = 730ull << 20;
+constexpr uint64_t kSpeciesStream = 420ull << 20, kSpeciesStream64 = 560ull << 20;
 
-template <int D, class T, bool FUSED>
+enum AdrLaunch { kFusedStep, kReactionStep, kScalarStep };
+
+template <int D, class T, AdrLaunch L>
 Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t fluid, uint64_t species) {
+    constexpr bool fused = L == kFusedStep;
     const uint64_t plane = s.cells.count, bytes = plane * sizeof(T), loop = (fluid + species) * bytes;
     Traffic t = plan_traffic<D, T>(s, bases, plane, loop);
     if (tiled || wide_planes<T>(s)) {
         t = Traffic{true, kDispatchOrder};
     } else if (loop > kCachedBytes) {
         const uint64_t q = crowding(bytes, fluid + species);
-        const bool crowded = q != 0 && loop <= (FUSED || D == 2 ? kCrowdedBytes : kCrowdedSpecies);
+        const bool crowded = q != 0 && loop <= (fused || D == 2 ? kCrowdedBytes : kCrowdedSpecies);
         t.order = large_order<D, T>(t.streaming, plane);
         if (crowded && (D == 2 || t.streaming))
             t.order = D == 3 && sizeof(T) == 2 && q < 3 ? kDispatchOrder : kContiguousOrder;
-        if (!FUSED && D == 2) {
+        if (!fused && D == 2) {
             if (t.streaming && fluid * bytes <= kContiguousBytes) t.order = kContiguousOrder;
+            if (!t.streaming && ((crowded && L == kScalarStep) || loop <= kSpeciesStream))
+                t = Traffic{true, kContiguousOrder};
+            if (!t.streaming && L == kScalarStep && sizeof(T) == 8 && loop <= kSpeciesStream64)
+                t = Traffic{true, kDispatchOrder};
         }
-        if (!FUSED && D == 3 && t.streaming && !crowded && (sizeof(T) == 2 || (sizeof(T) == 8 && loop > kSpeciesRuns)))
+        if (!fused && D == 3 && t.streaming && !crowded && (sizeof(T) == 2 || (sizeof(T) == 8 && loop > kSpeciesRuns)))
             t.order = kDispatchOrder;
     }
     s.cells.order = t.order;

@@ -96,3 +96,13 @@ def test_3d_species_steps_in_dispatch_order(plans):
                  ("f16", (320, 320, 320), DISPATCH), ("f16", (168, 168, 168), DISPATCH), ("f32", (192, 192, 192), DISPATCH),
                  ("f64", (128, 128, 128), CONTIGUOUS)]
         assert plans([(step, st, e, 19, 0) for st, e, _ in cases]) == [(True, order) for *_, order in cases], step
+
+
+def test_misaligned_2d_species_steps_stream_while_that_pays(plans):
+    cases = [("reaction", "f32", (1501, 1501, 1), (True, CONTIGUOUS)), ("scalar", "f32", (1801, 1799, 1), (True, CONTIGUOUS)),
+             ("reaction", "f64", (1201, 1199, 1), (True, CONTIGUOUS)), ("scalar", "f32", (2049, 2047, 1), (True, CONTIGUOUS)),
+             ("scalar", "f64", (1449, 1447, 1), (True, CONTIGUOUS)),
+             ("reaction", "f64", (1449, 1447, 1), (False, CONTIGUOUS)), ("reaction", "f64", (1301, 1299, 1), (False, RUNS_OF_32)), ("scalar", "f64", (1501, 1499, 1), (True, DISPATCH)),
+             ("reaction", "f32", (1951, 1949, 1), (False, RUNS_OF_32)), ("scalar", "f32", (2201, 2199, 1), (False, RUNS_OF_32)),
+             ("scalar", "f64", (1701, 1699, 1), (False, RUNS_OF_32)), ("reaction", "f32", (1001, 701, 1), (False, CONTIGUOUS))]
+    assert plans([(step, st, e, 9, 0) for step, st, e, _ in cases]) == [want for *_, want in cases]

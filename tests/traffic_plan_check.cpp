@@ -13,9 +13,9 @@
 
 template <int D, class T> lbc::Traffic plan(const char* step, lbc::LaunchShape& s, int q, uint64_t base) {
     const uint64_t qs = D == 2 ? 5 : 7;
-    if (std::strcmp(step, "fused") == 0) return lbc::adr_traffic<D, T, true>(s, false, base, 2 * q, 4 * qs);
-    if (std::strcmp(step, "reaction") == 0) return lbc::adr_traffic<D, T, false>(s, false, base, 2 * q, 4 * qs);
-    if (std::strcmp(step, "scalar") == 0) return lbc::adr_traffic<D, T, false>(s, false, base, 2 * q, 2 * qs);
+    if (std::strcmp(step, "fused") == 0) return lbc::adr_traffic<D, T, lbc::kFusedStep>(s, false, base, 2 * q, 4 * qs);
+    if (std::strcmp(step, "reaction") == 0) return lbc::adr_traffic<D, T, lbc::kReactionStep>(s, false, base, 2 * q, 4 * qs);
+    if (std::strcmp(step, "scalar") == 0) return lbc::adr_traffic<D, T, lbc::kScalarStep>(s, false, base, 2 * q, 2 * qs);
     return lbc::plan_traffic<D, T>(s, base, s.cells.count, 2ull * q * s.cells.count * sizeof(T));
 }
 
