@@ -336,13 +336,25 @@ constexpr uint64_t kContiguousBytes = 296ull << 20;
 // 512 x 256 3.46-4.03 against 3.57-4.01).
 constexpr uint64_t kPlanesInStep = 256ull << 20;
 
+// 16-bit planes within 128 KiB of a small multiple of 4 MiB lose in runs too
+// (D3Q19 TRT FP16 / BF16, runs of 8 over dispatch order in three placements: 8 MiB
+// 1.06-1.14 / 1.04-1.18, 11.9 1.09-1.13 / 1.00-1.07, 12 1.03-1.07, 16 1.04 / 1.05, 20
+// 1.01-1.04 / 1.00-1.06, 24 0.99-1.07 / 0.98-1.04; D3Q27 FP16 8 MiB 1.03-1.08, 12
+// 1.00-1.03; between them, 7.75 to 23 MiB, 0.97-0.99, and 28 MiB and more 0.96-0.99).
+constexpr uint64_t kStepNear = 128ull << 10, kStepMost = 25ull << 20;
+
+inline bool planes_in_step(uint64_t bytes, uint64_t element) {
+    constexpr uint64_t kStep = 4ull << 20;
+    if (element == 2 && bytes + kStepNear >= kStep && bytes < kStepMost && (bytes + kStepNear) % kStep <= 2 * kStepNear)
+        return true;
+    return bytes % kPlanesInStep == 0 && (element == 2 || bytes == kPlanesInStep);
+}
+
 // The order past the caches, of planes `plane` elements apart.
 template <int D, class S> uint32_t large_order(bool streaming, uint64_t plane) {
     if (!streaming) return 5u;
     if (D == 2) return sizeof(S) <= 4 ? 3u : kDispatchOrder;
-    const uint64_t bytes = plane * sizeof(S);
-    const bool in_step = bytes % kPlanesInStep == 0 && (sizeof(S) == 2 || bytes == kPlanesInStep);
-    return sizeof(S) == 4 || in_step ? kDispatchOrder : 3u;
+    return sizeof(S) == 4 || planes_in_step(plane * sizeof(S), sizeof(S)) ? kDispatchOrder : 3u;
 }
 
 template <int D, class S>

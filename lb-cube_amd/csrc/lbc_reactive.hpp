@@ -193,9 +193,8 @@ inline uint64_t crowding(uint64_t plane_bytes, uint64_t planes) {
 //    -> 149; D3Q27 FP32 120^3 106 -> 117.
 //  - crowded past the limit: 2048 x 4096 FP32 229 -> 241; D3Q19 FP16 192 x 256 x
 //    128 161 -> 170, FP32 256 x 128 x 128 195-198 -> 194-204.
-//  - 3D at 2 bytes, where q < 3 gains nothing and the runs lose: in dispatch order
-//    (TRT FP16 256 x 256 x 64 100 us, contiguous 101, runs of 8 103; BF16 512 x 128 x
-//    64 108, 109 and 114).
+//  - 3D at 2 bytes, where q < 3 gains nothing: in dispatch order (TRT FP16 256 x
+//    256 x 64 100 us, contiguous 101; BF16 512 x 128 x 64 108 and 109).
 constexpr uint64_t kCrowdedBytes = 730ull << 20;
 
 // The launch of the species alone reads what the fluid's launch has left.  2D:
@@ -233,8 +232,7 @@ Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t fluid, 
         const uint64_t q = crowding(bytes, fluid + species);
         const bool crowded = q != 0 && loop <= (fused || D == 2 ? kCrowdedBytes : kCrowdedSpecies);
         t.order = large_order<D, T>(t.streaming, plane);
-        if (crowded && (D == 2 || t.streaming))
-            t.order = D == 3 && sizeof(T) == 2 && q < 3 ? kDispatchOrder : kContiguousOrder;
+        if (crowded && (D == 2 || (t.streaming && (sizeof(T) > 2 || q > 2)))) t.order = kContiguousOrder;
         if (!fused && D == 2) {
             if (t.streaming && fluid * bytes <= kContiguousBytes) t.order = kContiguousOrder;
             if (!t.streaming && ((crowded && L == kScalarStep) || loop <= kSpeciesStream))

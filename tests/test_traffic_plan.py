@@ -68,7 +68,7 @@ def test_fused_steps_run_contiguously_only_where_their_planes_crowd_the_cache_se
               ("f16", (168, 168, 168), (True, RUNS_OF_8)), ("f64", (104, 104, 104), (True, RUNS_OF_8)),
               # crowded, but past the limit, or at two bytes in one or two groups
               ("f32", (2048, 4096, 1), (True, RUNS_OF_8)), ("f32", (256, 128, 128), (True, DISPATCH)),
-              ("f16", (192, 256, 128), (True, RUNS_OF_8)), ("f16", (256, 256, 64), (True, DISPATCH))]
+              ("f16", (192, 256, 130), (True, RUNS_OF_8)), ("f16", (256, 256, 64), (True, DISPATCH))]
     assert plans([("fused", st, e, 9 if e[2] == 1 else 19, 0) for st, e, _ in spread]) == [want for *_, want in spread]
     cached = [("f32", (512, 512, 1)), ("f32", (1001, 701, 1)), ("f64", (64, 64, 64)), ("f32", (96, 96, 96))]
     got = plans([("fused", st, e, 9 if e[2] == 1 else 19, 0) for st, e in cached])
@@ -106,3 +106,18 @@ def test_misaligned_2d_species_steps_stream_while_that_pays(plans):
              ("reaction", "f32", (1951, 1949, 1), (False, RUNS_OF_32)), ("scalar", "f32", (2201, 2199, 1), (False, RUNS_OF_32)),
              ("scalar", "f64", (1701, 1699, 1), (False, RUNS_OF_32)), ("reaction", "f32", (1001, 701, 1), (False, CONTIGUOUS))]
     assert plans([(step, st, e, 9, 0) for step, st, e, _ in cases]) == [want for *_, want in cases]
+
+
+def test_16_bit_planes_near_small_multiples_of_4_mib_keep_the_dispatch_order(plans):
+    near = [(256, 256, 63), (256, 256, 64), (128, 128, 256), (256, 256, 65), (192, 256, 128), (256, 256, 95),
+            (256, 256, 128), (256, 256, 160), (256, 256, 192)]
+    others = [(256, 256, 62), (256, 256, 66), (256, 256, 80), (256, 256, 126), (256, 256, 176), (256, 256, 224),
+              (256, 256, 256), (320, 320, 320)]
+    for q in (19, 27):
+        assert plans([("fluid", "f16", e, q, 0) for e in near]) == [(True, DISPATCH)] * len(near)
+        assert plans([("fluid", "f16", e, q, 0) for e in others]) == [(True, RUNS_OF_8)] * len(others)
+    wide = [("f64", (128, 128, 64), RUNS_OF_8), ("f32", (256, 128, 64), DISPATCH)]
+    assert plans([("fluid", st, e, 19, 0) for st, e, _ in wide]) == [(True, order) for *_, order in wide]
+    # slabs of 128 and 512 KiB are no planes 4 MiB apart
+    slabs = [("f16", (256, 256, 256)), ("f16", (512, 512, 512)), ("f64", (256, 256, 256))]
+    assert plans([("slabs", st, e, 19, 0) for st, e in slabs]) == [(True, RUNS_OF_8)] * 3

@@ -1,8 +1,9 @@
 // Host check of the steps' store form and block order (the rules of
 // lb-cube_amd/csrc/lbc_launch.hpp and lbc_reactive.hpp, the headers' own code).
 // Each line of stdin is "<step> <element bytes> <nx> <ny> <nz> <Q> <offset>":
-// step is fluid, fused, reaction or scalar, Q the fluid's; the planes of a domain
-// lie back to back, `offset` bytes past a cache line (nz = 1: 2D).
+// step is fluid, slabs (the fluid step in the slab order), fused, reaction or
+// scalar, Q the fluid's; the planes of a domain lie back to back, `offset` bytes
+// past a cache line (nz = 1: 2D).
 // Prints "<streaming> <order>" for each.
 #include <cstdint>
 #include <cstdio>
@@ -16,6 +17,11 @@ template <int D, class T> lbc::Traffic plan(const char* step, lbc::LaunchShape& 
     if (std::strcmp(step, "fused") == 0) return lbc::adr_traffic<D, T, lbc::kFusedStep>(s, false, base, 2 * q, 4 * qs);
     if (std::strcmp(step, "reaction") == 0) return lbc::adr_traffic<D, T, lbc::kReactionStep>(s, false, base, 2 * q, 4 * qs);
     if (std::strcmp(step, "scalar") == 0) return lbc::adr_traffic<D, T, lbc::kScalarStep>(s, false, base, 2 * q, 2 * qs);
+    if (std::strcmp(step, "slabs") == 0) {
+        const uint64_t cells = s.cells.count, slab = cells / s.cells.nz;
+        s.cells.zgap = static_cast<uint32_t>((q - 1) * slab);
+        return lbc::plan_traffic<D, T>(s, base, slab, 2ull * q * cells * sizeof(T));
+    }
     return lbc::plan_traffic<D, T>(s, base, s.cells.count, 2ull * q * s.cells.count * sizeof(T));
 }
 
