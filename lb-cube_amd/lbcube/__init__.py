@@ -44,8 +44,11 @@ SCALAR_PAIRS = {("D2Q9", "D2Q5"), ("D3Q19", "D3Q7"), ("D3Q27", "D3Q7")}
 
 
 def _stream(stream):
-    if stream is None:  # torch.cuda.current_stream().cuda_stream without the Stream object
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if stream is None:
+        try:  # torch.cuda.current_stream().cuda_stream without the Stream object
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        except AttributeError:  # private names, which another torch may not have
+            return torch.cuda.current_stream().cuda_stream
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 

@@ -2,6 +2,8 @@
 and a call without a stream runs on torch's current one."""
 from __future__ import annotations
 
+import types
+
 import pytest
 import torch
 
@@ -23,3 +25,10 @@ def test_current_stream_is_torch_s(gpu):
     with torch.cuda.stream(side):
         assert lbcube._stream(None) == side.cuda_stream == lbcube._stream(side)
     assert lbcube._stream(None) == torch.cuda.current_stream().cuda_stream
+
+
+@pytest.mark.parametrize("name", ["_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_current_stream_without_torchs_private_names(monkeypatch, name):
+    monkeypatch.delattr(torch._C, name, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
+    assert lbcube._stream(None) == 77
