@@ -951,6 +951,28 @@ def cpu_baseline(u_host, omega, n):
             "single_thread_value": cells / t_one / 1e6, "host_cpus": os.cpu_count(), "cpu_model": model}
 
 
+# What a rate's MLUPS, its storage and lattice determine, and the runs' checks:
+# left out of the printed line.
+DERIVED = {"achieved_gbs", "roofline_frac", "bytes_per_cell", "ms_per_step", "cells", "plane_bytes", "final_mass",
+           "final_ke", "unfused_achieved_gbs", "unfused_bytes_per_cell"}
+
+
+def compact(record):
+    """`record` with five significant digits and each rate without what follows
+    from its MLUPS (a bare number where nothing else is left)."""
+    if isinstance(record, dict):
+        kept = {k: compact(v) for k, v in record.items() if not ("mlups" in record and k in DERIVED)}
+        return kept["mlups"] if list(kept) == ["mlups"] else kept
+    return float(f"{record:.5g}") if isinstance(record, float) else record
+
+
+def headline(out):
+    """The printed line: the headline in full and its configurations compacted,
+    so that it stays short enough to be read whole from a log's tail."""
+    groups = ("variants", "pitched_planes", "configs")
+    return json.dumps({k: compact(v) if k in groups else v for k, v in out.items()}, separators=(",", ":"))
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -966,6 +988,7 @@ def main():
     ap.add_argument("--no-extras", action="store_true", help="skip the adjoint, ensemble and 2D reactive lines")
     ap.add_argument("--extras", default="pitched,adjoint,reactive_2d,adr_3d,ensemble,lattices,large,tiles_3d,shard",
                     help="which configuration lines to run (comma-separated subset)")
+    ap.add_argument("--details", default=None, metavar="FILE", help="write the whole record there as JSON")
     args = ap.parse_args()
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
@@ -1090,7 +1113,10 @@ def main():
         if "adjoint" in extras:
             out["adjoint_over_forward"] = round(extras["adjoint"]["adjoint_over_forward"], 3)
         out["configs"] = extras
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as fh:
+            json.dump(out, fh)
+    print(headline(out))
 
 
 if __name__ == "__main__":
