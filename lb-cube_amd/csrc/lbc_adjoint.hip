@@ -389,10 +389,11 @@ __global__ __launch_bounds__(MAXT) void reactive_trace_kernel(
 // into LDS, and the second on the tile without its rim, so the fluid between
 // the two steps never leaves the chip and half the launches go.  A single step
 // of the domains that stay in the caches is a chain of latencies (launch, loads,
-// stores) more than traffic; the rims repeat 1.22 of the first step.  Gradients,
-// single steps -> pairs: FP32 512^2, 1024 steps, 24.85 -> 21.95 ms; 200^2, 400
-// steps, 4.14 -> 3.66; 600^2, 400 steps, 13.0 -> 11.2; FP64 512^2, 200 steps, 8.35
-// -> 7.47.  Tiles of 32 rows: 23.6 for the first (two blocks per CU); the blocks
+// stores) more than traffic; the rims repeat 1.22 of the first step.  Gradients
+// in the deviation form, single steps -> pairs, each in its own schedule
+// (overlapped): FP32 512^2, 1024 steps, 24.85 -> 21.95 ms; 200^2, 400 steps, 4.68 ->
+// 3.67; 600^2, 300 steps, 9.9 -> 8.6; FP64 512^2, 200 steps, 9.1 -> 7.9; MRT 131^2,
+// 400 steps, 5.09 -> 4.57.  Tiles of 32 rows: 23.6 for the first (two blocks per CU); the blocks
 // in dispatch order 26.9, in runs of 8 22.9 (neighbouring tiles share lines).
 // The same values as two single steps: the tile holds the populations as the
 // single step stores them.  macro0 with mid_a and mid_b (the trace of the first
@@ -906,11 +907,14 @@ hipError_t run_gradient(uint32_t flags, const R* f0, const R* a0, const R* b0, c
                                                                   s.block.y, s.block.z, on));
     };
     // two forward steps in one launch (kPair); mid.f is not written
-    // Not in the reference's order on small domains: its steps are bound by their
-    // arithmetic, which the rims repeat, on too few tiles for 256 CUs (D2Q9 MRT
-    // FP32 at 333^2, 400 steps: 5.65 ms in single steps, 6.0 in pairs; BGK FP64 at
-    // 600^2, 200 steps: 11.1 and 9.9).  Nor past the caches, where the tiles' short
-    // rows leave partial lines (FP32 at 2048^2, 40 steps: 13.2 and 17.2).
+    // In the reference's order from kPairCells on: its steps are bound by their
+    // arithmetic, which the rims repeat, and just past one tile per CU the last
+    // tiles run alone (TRT FP32, 400 steps: 333^2 5.89 ms in single steps, 6.21 in
+    // pairs, 400^2 7.32 and 7.05; FP64 360^2 9.39 and 9.59; BGK FP64 600^2, 200
+    // steps, 11.1 and 9.9).  Below, down to one tile per CU, pairs would gain too
+    // (TRT FP32 200^2 5.05 and 3.90); the single steps that the pairs are tested
+    // against stay there.  Nor past the caches, where the tiles' short rows leave
+    // partial lines (FP32 at 2048^2, 40 steps: 13.2 and 17.2).
     constexpr bool kPair = kTrace && F::D == 2;
     constexpr size_t kPairCells = 1u << 18;
     const bool pairs = kPair && 2 * se * sizeof(R) <= kCachedBytes &&

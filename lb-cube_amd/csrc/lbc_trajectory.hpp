@@ -58,9 +58,10 @@ inline std::size_t trajectory_capacity(std::size_t state, std::size_t steps, std
 // states below kShortState32 (FP64: kShortState64) need segments of
 // kShortSteps (RLBM FP32 400 steps, interval 16: 128^2 5.15 and 4.53, 200^2 4.92
 // and 4.91, 240^2 4.75 and 5.17; interval 32, 1024 steps: 128^2 12.1 and 13.0;
-// FP64, interval 16: 16^2 5.01 and 4.71, 24^2 5.03 and 5.33).
+// FP64, interval 16: TRT 32^2 5.33 and 5.01, 64^2 5.23 and 5.25, RLBM 32^2 5.42 and
+// 5.33, 64^2 5.34 and 5.56).
 constexpr std::size_t kOverlapSteps = 8, kShortSteps = 32, kOverlapMax = 40u << 20;
-constexpr std::size_t kShortState32 = 4u << 20, kShortState64 = 64u << 10;
+constexpr std::size_t kShortState32 = 4u << 20, kShortState64 = 256u << 10;
 
 // state_bytes: of one state of `element`-byte populations; paired: two steps
 // per launch.

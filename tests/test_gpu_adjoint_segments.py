@@ -16,7 +16,7 @@ from schedules import schedule
 
 STEPS = 40
 # fluid lattice, extents (x first), blocks: small and larger than one block, the default and the 1024-work-item kernels
-DOMAINS = [("D2Q9", (12, 10), (None, (1024, 1, 1))), ("D2Q9", (40, 30), (None, (32, 32, 1))),
+DOMAINS = [("D2Q9", (12, 10), (None, (1024, 1, 1))), ("D2Q9", (60, 50), (None, (32, 32, 1))),
            ("D3Q19", (7, 6, 5), (None, (1024, 1, 1))), ("D3Q19", (12, 10, 9), (None, (16, 16, 4))),
            ("D3Q27", (7, 6, 5), (None, (16, 16, 4)))]
 

@@ -46,7 +46,8 @@ def test_states_that_leave_the_gpu_idle_are_overlapped():
     assert not schedule("D2Q9", (128, 128), "RLBM", "f32", 400, 16).overlapped
     assert schedule("D2Q9", (240, 240), "RLBM", "f32", 400, 16).overlapped
     assert schedule("D2Q9", (128, 128), "RLBM", "f32", 1024, 32).overlapped
-    assert not schedule("D2Q9", (16, 16), "RLBM", "f64", 400, 16).overlapped
+    assert not schedule("D2Q9", (32, 32), "TRT", "f64", 400, 16).overlapped
+    assert schedule("D2Q9", (48, 48), "TRT", "f64", 400, 16).overlapped
     assert not schedule("D2Q9", (1024, 1024), "BGK", "f32", 256, 16, True).overlapped
     assert not schedule("D2Q9", (200, 200), "BGK", "f32", 23, 3, True).overlapped
     assert not schedule("D2Q9", (200, 200), "BGK", "f32", 40, 40, True).overlapped
