@@ -1,7 +1,7 @@
 """GPU: the discrete adjoint of the 2D reactive loop (lbc_reactive_gradient).
 
-  * against the oracle's FP64 CPU adjoint (tight tolerance, several checkpoint
-    intervals so the segment recompute is exercised);
+  * against the oracle's FP64 CPU adjoint (tight tolerance, several workspaces;
+    runs that are cut into segments: test_gpu_adjoint_segments.py);
   * checkpoint-interval invariance: recomputed segments are bit-identical, so
     every interval gives the same gradient bit for bit;
   * torch.autograd.gradcheck of the autograd wrapper in FP64 on a tiny grid;
@@ -29,8 +29,8 @@ def dev(x, gpu, dtype=torch.float64):
 @pytest.mark.parametrize("coll", ["BGK", "TRT", "MRT", "RLBM"])
 @pytest.mark.parametrize("interval", [1, 5, 8, 64])
 def test_adjoint_matches_oracle_fp64(gpu, coll, interval):
-    # interval 8 over 17 steps: three segments (8, 8, 1), the recomputes
-    # overlapped with the adjoint walks on a second stream
+    # the workspace holds the whole run, but for RLBM at interval 5 (three
+    # segments)
     print(f"case adjoint {coll} interval={interval}", flush=True)
     f, a, b = TA.small_state(nx=12, ny=10, seed=4)
     omega, omega_c, k, steps = 1 / 0.7, 1 / 0.9, 0.4, 17
@@ -111,8 +111,8 @@ def test_checkpoint_interval_invariance(gpu):
     f, a, b = TA.small_state(nx=64, ny=48, seed=2)
     args = (dev(f, gpu), dev(a, gpu), dev(b, gpu), 50, 1 / 0.6, 1 / 0.8, 0.05)
     ref = ADJ.reactive_gradient("BGK", *args, interval=50)
-    # 1 and 7: every segment on one stream; 8 and 16: recomputes overlapped
-    # with the adjoint walks (interval >= 8 and more than one segment)
+    # 1, 16 and 64: one segment; 7 and 8: five and four segments of 12 and 13
+    # steps, the recomputes overlapped with the adjoint walks
     for interval in (1, 7, 8, 16, 64):
         got = ADJ.reactive_gradient("BGK", *args, interval=interval)
         assert got[0] == ref[0] and got[4] == ref[4]

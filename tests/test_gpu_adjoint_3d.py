@@ -2,8 +2,8 @@
 a D3Q19 or D3Q27 fluid (BGK, TRT, MRT, RLBM) with two D3Q7 species, A + B -> C.
 
   * against the oracle's FP64 CPU adjoint of the same loop (tight tolerance;
-    checkpoint intervals 1, 5 and 8 over 17 steps, so the segment recompute
-    and its overlap with the adjoint walk are exercised);
+    several workspaces, which hold the 17 steps but for RLBM at interval 5; runs
+    that are cut into segments: test_gpu_adjoint_segments.py);
   * blocks of 1024 work-items (the kernels' second instantiation), 2D and 3D,
     every collision, against the same oracle;
   * the FP32 adjoint, and the FP64 adjoint of the FP32 trajectory, against the
@@ -55,7 +55,7 @@ def test_adjoint_3d_matches_oracle_fp64(gpu, lattice, coll, interval):
 def test_adjoint_blocks_of_1024_match_oracle(gpu, lattice, coll):
     """The kernels' 1024-work-item instantiations (the largest block the
     reference's launchers accept; they spill registers to scratch) against
-    the oracle's FP64 adjoint, with checkpoints every 5 steps: blocks of
+    the oracle's FP64 adjoint, in one segment: blocks of
     1024 x 1 x 1 and, in 3D, 16 x 16 x 4."""
     print(f"case adjoint blocks of 1024 {lattice} {coll}", flush=True)
     if lattice == "D2Q9":

@@ -33,8 +33,8 @@ def state(lattice, shape, dtype, gpu):
             lbinit.scalar_equilibrium(species, 1.0 - c, u, dtype))
 
 
-# intervals whose plans have one segment, two, and more of fewer and of more
-# than eight steps (recomputes on one stream and on two), with short first ones
+# intervals whose plans have one segment and more, of fewer and of more than
+# eight steps (recomputes on one stream and on two), with short first ones
 CASES = [("D2Q9", (13, 37), "MRT", "f32", False, (1, 4, 5, 7)), ("D2Q9", (32, 64), "TRT", "f64", False, (1, 5, 6)),
          ("D3Q19", (5, 9, 11), "TRT", "f32", False, (1, 3, 4, 6)), ("D3Q19", (8, 8, 16), "MRT", "f64", False, (2, 5)),
          ("D3Q27", (6, 7, 9), "BGK", "f32", False, (2, 5)), ("D3Q27", (6, 7, 9), "MRT", "f32", False, (2, 5)),
