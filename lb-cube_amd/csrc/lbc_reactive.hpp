@@ -202,11 +202,12 @@ constexpr uint64_t kCrowdedBytes = 730ull << 20;
 // 1472^2, loop of two launches: both contiguous 143.6 us, both in dispatch
 // order 139.7, one of each 148.8).  3D: contiguous where crowded up to
 // kCrowdedSpecies (D3Q19 FP32 256 x 128 x 128 247-257 -> 239-247, FP64 128^3
-// 253-275 -> 242-253).  Else FP64 in runs up to kSpeciesRuns (120^3 214.8 ->
-// 210.5) and in dispatch order above (256^3 2028-2046, in runs of 8 2081-2098;
-// 256 x 256 x 192 1578 and 1681), 2-byte storage in dispatch order (FP16 320^3
-// 1004-1018, in runs 1058-1075, with two scalars 1215 and 1271; from 144^3 to
-// 416^3 else within 2% either way).
+// 253-275 -> 242-253).  Else FP64 in runs of 8 up to kSpeciesRuns64 (120^3 214.8
+// -> 210.5) and in dispatch order above (256^3 2028-2046, in runs 2081-2098; 256 x
+// 256 x 192 1578 and 1681), FP32 so with kSpeciesRuns32 (104^3 61.1 -> 59.6, two
+// scalars at 120^3 112 -> 107; 128 x 128 x 112 110.5 and 111.7), 2-byte storage in
+// dispatch order (FP16 320^3 1004-1018, in runs 1058-1075, with two scalars 1215
+// and 1271; from 144^3 to 416^3 else within 2% either way).
 // Misaligned 2D planes: streaming stores leave the fluid in the caches.
 // Contiguous up to kSpeciesStream (ordinary -> streaming: two scalars FP32 1801
 // x 1799 120 -> 115, FP64 1301 x 1299 129 -> 121; reaction FP64 1201 x 1199 107 ->
@@ -216,7 +217,7 @@ constexpr uint64_t kCrowdedBytes = 730ull << 20;
 // to kSpeciesStream64 (1501 x 1499 181 -> 173, 1551 x 1549 194 -> 185; not the
 // reaction step: 1301 x 1299 118 -> 123, nor FP32 and FP16: 2401 x 2399 240 -> 248,
 // 3001 x 2999 189 -> 195).
-constexpr uint64_t kCrowdedSpecies = 1100ull << 20, kSpeciesRuns = 730ull << 20;
+constexpr uint64_t kCrowdedSpecies = 1100ull << 20, kSpeciesRuns64 = 730ull << 20, kSpeciesRuns32 = 450ull << 20;
 constexpr uint64_t kSpeciesStream = 420ull << 20, kSpeciesStream64 = 560ull << 20;
 
 enum AdrLaunch { kFusedStep, kReactionStep, kScalarStep };
@@ -240,8 +241,10 @@ Traffic adr_traffic(LaunchShape& s, bool tiled, uint64_t bases, uint64_t fluid, 
             if (!t.streaming && L == kScalarStep && sizeof(T) == 8 && loop <= kSpeciesStream64)
                 t = Traffic{true, kDispatchOrder};
         }
-        if (!fused && D == 3 && t.streaming && !crowded && (sizeof(T) == 2 || (sizeof(T) == 8 && loop > kSpeciesRuns)))
-            t.order = kDispatchOrder;
+        if (!fused && D == 3 && t.streaming && !crowded) {
+            constexpr uint64_t runs = sizeof(T) == 8 ? kSpeciesRuns64 : sizeof(T) == 4 ? kSpeciesRuns32 : 0;
+            t.order = loop <= runs ? 3u : kDispatchOrder;
+        }
     }
     s.cells.order = t.order;
     return t;

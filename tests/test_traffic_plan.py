@@ -94,6 +94,7 @@ def test_3d_species_steps_in_dispatch_order(plans):
     for step in ("reaction", "scalar"):
         cases = [("f64", (256, 256, 256), DISPATCH), ("f64", (256, 256, 192), DISPATCH), ("f64", (104, 104, 104), RUNS_OF_8),
                  ("f16", (320, 320, 320), DISPATCH), ("f16", (168, 168, 168), DISPATCH), ("f32", (192, 192, 192), DISPATCH),
+                 ("f32", (120, 120, 120), RUNS_OF_8), ("f32", (144, 136, 144), DISPATCH),
                  ("f64", (128, 128, 128), CONTIGUOUS)]
         assert plans([(step, st, e, 19, 0) for st, e, _ in cases]) == [(True, order) for *_, order in cases], step
 
